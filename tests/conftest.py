@@ -28,3 +28,20 @@ def small_case():
     D = A.todense()
     s = np.linalg.svd(D, compute_uv=False)
     return A, u0, D, s
+
+
+@pytest.fixture(autouse=True, scope="session")
+def _reference_or_skip():
+    """A test that runs the compiled reference skips where the reference was
+    not built (its sources are not on every machine); loading it there would
+    end the test with an OSError from the dynamic loader."""
+    from oracle import refpy
+    load = refpy.lib
+
+    def lib(prec="d"):
+        if not refpy.available(prec):
+            pytest.skip(f"oracle/_ref/libpropack_ref_{prec}.so is not built")
+        return load(prec)
+    refpy.lib = lib
+    yield
+    refpy.lib = load
