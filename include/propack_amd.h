@@ -98,6 +98,15 @@ int pk_csr_spmv(pk_csr_t op, char trans, const void* x, void* y, int prec, int w
  * the switch keeps the panel-by-panel path).
  * Row sums are bit-identical to the row-block layout's for the same lanes;
  * only the per-block partial sums of the norms are grouped differently.
+ * A direction of at least 2^22 nonzeros runs in the tile layout instead --
+ * row sums accumulated in LDS while its nonzeros stream past in column order;
+ * equal up to rounding, bit-identical run to run -- when no layout was asked
+ * for at creation, and in place of every panel in one launch; its rows must
+ * be even (long or uneven rows keep the other layouts).  The settings are
+ * reported as they were asked.  It takes another 12 bytes per nonzero
+ * (8 for FP32 values) and up to 16 FP64 sums per row per operator and
+ * engine; batches run such an operator's panels, and an engine created
+ * before the switch too.
  * Not while a solve that uses the operator runs.  A batch (pk_batch_create)
  * takes the layout its operators have when it is created; once an
  * operator's lanes or sorted layout change, the batch's calls fail with
@@ -169,7 +178,8 @@ int pk_csr_to_iparm(pk_csr_t op, int* iparm);
  * long-row sums go to a fixed 48 MiB device array per GPU, set up on the
  * first call on each device; an operator needing more (about 6M rows in a
  * multi-panel direction) is refused with PK_ERR_NOTSUP.  Results are
- * bit-identical to pk_csr_spmv's.  Calls that overlap on one GPU share that
+ * bit-identical to pk_csr_spmv's (to rounding where a tile layout's row sums
+ * do not fit beside the partial sums: more than about 10^9 nonzeros).  Calls that overlap on one GPU share that
  * array and race: order them on one stream. */
 int pk_csr_spmv_noalloc(pk_csr_t op, char trans, const void* x, void* y, int prec,
                         void* stream);

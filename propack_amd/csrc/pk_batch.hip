@@ -588,7 +588,7 @@ int batch_create(int nprob, const pk_lbd_t* handles, Batch** out) {
     B->maxk = std::max(B->maxk, e->kmax);
     B->rstride = std::max(B->rstride, e->ccap);
     for (int tr = 0; tr < 2 && rc == PK_OK; ++tr) {
-      const CsrOp::Dir& D = tr ? e->op->dt : e->op->da;
+      CsrOp::Dir& D = tr ? e->op->dt : e->op->da;
       (tr ? P.npt : P.npa) = D.np;
       // the engine's own scratch: the SpMVs of both directions run one after
       // the other on the batch's stream
@@ -596,7 +596,7 @@ int batch_create(int nprob, const pk_lbd_t* handles, Batch** out) {
       // the layout the operator uses for this direction (row-block,
       // row-wise over the row-block arrays (cap -1), or column-sorted),
       // exactly as its own SpMV runs it
-      const int cap = D.rowwise ? -1 : D.sort_cap;
+      const int cap = D.rowwise ? -1 : csr_ensure_sorted(e->op, D) ? D.sort_cap : 0;
       for (int p = 0; p < D.np; ++p) {
         const CsrOp::Panel& pan = D.pan[p];
         const CsrOp::Part& part = cap > 0 ? pan.spart : pan.part;

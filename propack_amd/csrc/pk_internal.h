@@ -10,6 +10,33 @@
 
 namespace pk {
 
+// Tile layout of one direction (pk_tile.hip): units of (row tile, column
+// segment), each a run of batches of kTileThreads entries with distinct rows.
+constexpr int kTileThreads = 1024;
+constexpr int kTileRows = 20000;  // FP64 row sums of a tile: 160,000 of 163,840 LDS bytes
+constexpr int kMaxTileSegs = 16;
+constexpr double kTileImbalance = 1.25;  // largest unit over the mean one
+struct TileDesc {
+  int row0, nrows, b0, nb;  // rows, first batch, batches
+  int seg, pad0, pad1, pad2;
+};
+struct TileLayout {
+  int nunit = 0;  // 0: not built
+  int nseg = 1, maxrows = 0;
+  TileDesc* desc = nullptr;
+  int* base = nullptr;      // per batch: the column its offsets count from
+  unsigned* wd = nullptr;   // per entry: column offset and row in tile
+  void* va = nullptr;
+  double* ypart = nullptr;  // the operator's own row sums (nseg > 1)
+};
+// A CSR the layout is built from: column panels over all rows.
+struct TileSource {
+  const int* rp;
+  const int* ci;
+  const void* va;
+  long long nnz;
+};
+
 struct CsrOp {
   static constexpr unsigned kMagic = 0x504b4353u;  // "PKCS"
   static constexpr int kMaxPanels = 16;
@@ -57,6 +84,8 @@ struct CsrOp {
     int slots = 0;           // partial slots of the widest panel
     int lane_shift = 0;      // lanes per row = built-in choice * 2^lane_shift
     int sort_cap = 0;        // > 0: column-sorted layout, blocks of <= sort_cap nonzeros
+    int sorted = 0;          // the panels' sorted arrays are built (a direction in the tile
+                             // layout has sort_cap without them until a batch needs them)
     int rowwise = 0;         // row-block arrays summed row-wise, no LDS staging (k_spmv_vec)
     // column-sorted layout with every panel in one launch (np > 1): per-panel
     // FP64 row sums (np * rows doubles) combined in panel order afterwards
@@ -65,6 +94,9 @@ struct CsrOp {
     int2* cmap = nullptr;          // (panel, descriptor) of each workgroup
     int cmap_n = 0;
     double* ypart = nullptr;       // the operator's own per-panel row sums
+    // the layout of large directions (pk_tile.hip); when built it serves every
+    // application whose scratch holds its row sums
+    TileLayout tile;
   } da, dt;
   int nrb = 0, nrbt = 0;  // partial slots per direction
   // bumped by every layout change (lanes per row, sorted layout): a batch
@@ -116,6 +148,9 @@ int csr_sort_code(const CsrOp::Dir& D);
 // application needs (doubles): np * rows then, rows otherwise.
 bool csr_concurrent_ok(const CsrOp::Dir& D);
 long long csr_ywork(const CsrOp* op);
+// The sorted arrays of a direction with sort_cap > 0, built now if the tile
+// layout stood in for them; false if there are none.
+bool csr_ensure_sorted(CsrOp* op, CsrOp::Dir& D);
 // ywork (rows of the direction, doubles) and lwork (csr_lwork(op) doubles),
 // when given, replace the operator's own running row sums and long-row
 // partial sums, so that callers with their own scratch (every engine) may
@@ -129,6 +164,18 @@ int csr_apply(const CsrOp* op, hipStream_t s, char trans, const T* x, T* y, cons
 // Long-row partial sums one panel can need, for any layout of op: a row of
 // len > kSpmvCap nonzeros has ceil(len / kLongChunk) <= len / kSpmvCap chunks.
 inline long long csr_lwork(const CsrOp* op) { return op->nnz / 1024 + 2; }
+
+// ---- tile layout (pk_tile.hip) ----
+// Builds / frees a direction's tile layout; PK_ERR_NOTSUP (nothing built)
+// where rows are too long or too uneven for it.
+int tile_build(TileLayout& L, int rows, int cols, int val_prec, const TileSource* src, int nsrc,
+               hipStream_t s);
+void tile_free(TileLayout& L);
+// y = op(A) x - coef yprev from the tile layout; ypart: nseg * rows doubles
+// when nseg > 1.  Returns the partial-slot count.
+template <typename VT, typename T>
+int launch_spmv_tile(hipStream_t s, const TileLayout& L, long long rows, const T* x, T* y,
+                     const T* yprev, Scal coef, double* part, double* ypart, Gate gate);
 
 // ---- complex precisions (pk_cplx.hip) ----
 // A complex operator (val_prec PK_C128 / PK_C64) keeps A and the explicit

@@ -292,7 +292,11 @@ int launch_spmv_combine(hipStream_t s, long long rows, int np, const double* ypa
                      yprev, coef, y, part, gate)
   switch (np) {
     case 2: PK_CB_CASE(2); break;
+    case 3: PK_CB_CASE(3); break;
     case 4: PK_CB_CASE(4); break;
+    case 5: PK_CB_CASE(5); break;
+    case 6: PK_CB_CASE(6); break;
+    case 7: PK_CB_CASE(7); break;
     case 8: PK_CB_CASE(8); break;
     default: PK_CB_CASE(0); break;
   }
