@@ -566,12 +566,24 @@ struct Impl {
     PK_HIP(hipMemcpyAsync(e->dctl, static_cast<LbdCtl*>(&c), sizeof(LbdCtl),
                           hipMemcpyHostToDevice, strm));
     PK_HIP(hipMemcpyAsync(e->darr, e->harr, ab, hipMemcpyHostToDevice, strm));
-    for (int J = c.j; J <= c.k; ++J) PK_TRY(enqueue_step(J, elr, e->dev_tries));
+    // a small problem's steps run in one resident launch (class timing needs
+    // the chains' separate kernels)
+    int* const failed = reinterpret_cast<int*>(e->hred);
+    *failed = 0;
+    if (c.j <= kCtlLdsJ && !e->prof.on && resident_fits(e) && launch_resident<T>(e, strm) == 0) {
+      PK_HIP(hipMemcpyAsync(failed, &e->rbar->failed, sizeof(int), hipMemcpyDeviceToHost, strm));
+    } else {
+      for (int J = c.j; J <= c.k; ++J) PK_TRY(enqueue_step(J, elr, e->dev_tries));
+    }
     PK_HIP(hipMemcpyAsync(static_cast<LbdCtl*>(&c), e->dctl, sizeof(LbdCtl),
                           hipMemcpyDeviceToHost, strm));
     PK_HIP(hipMemcpyAsync(e->harr, e->darr, ab, hipMemcpyDeviceToHost, strm));
     PK_HIP(stream_wait(strm));
     e->cnt.nsync++;
+    if (*failed) {
+      set_error("resident Lanczos steps: a grid barrier did not complete");
+      return PK_ERR_HIP;
+    }
     // algorithmic bytes of the CGS passes the chain actually ran
     if (e->prof.on) {
       const double sb = static_cast<double>(sizeof(T));
@@ -1097,6 +1109,7 @@ static void engine_free(Engine* e) {
     (void)hipFree(e->V[i]);
   }
   (void)hipFree(e->part);
+  (void)hipFree(e->rbar);
   (void)hipFree(e->red);
   (void)hipFree(e->dcols);
   (void)hipFree(e->dB);
@@ -1181,7 +1194,9 @@ int pk_lbd_create(int prec, int m, int n, int kmax, pk_csr_t op, pk_lbd_t* out) 
   chk(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
   chk(hipMalloc(&e->U[0], e->tbytes * e->ldu * (kmax + 1)));
   chk(hipMalloc(&e->V[0], e->tbytes * e->ldv * kmax));
-  chk(hipMalloc(&e->part, sizeof(double) * nblk * e->ccap * cx));
+  e->part_len = nblk * e->ccap * cx;
+  chk(hipMalloc(&e->part, sizeof(double) * e->part_len));
+  chk(hipMalloc(&e->rbar, sizeof(ResidentBar)));
   chk(hipMalloc(&e->red, sizeof(double) * (e->ccap * cx + 16)));
   chk(hipMalloc(&e->dcols, sizeof(int) * e->ccap));
   chk(hipMalloc(&e->dB, sizeof(double) * nb));

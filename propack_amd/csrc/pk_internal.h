@@ -244,6 +244,41 @@ struct Counters {
   long long nwarn = 0;
 };
 
+// ---- resident steps of small problems (pk_resident.hip) ----
+struct ResidentBar {
+  unsigned count, pad0[31], passed, failed, pad1[30];
+  unsigned group[8 * 32];
+};
+struct ResidentDir {
+  const int4* desc;  // row blocks only (no long rows)
+  const int* rp;
+  const int* ci;
+  const void* va;
+  int ndesc, g;
+};
+constexpr int kResSlots = 2;   // row blocks of a direction per workgroup, held in LDS
+constexpr int kResGrid = 256;  // most workgroups (one per CU: they fill its LDS)
+struct ResidentArgs {
+  LbdCtl* ctl;
+  char* arrays;
+  int cap;
+  void* U;
+  void* V;
+  long long ldu, ldv;
+  int m, n;
+  double* part;    // two halves, used in turn
+  long long half;
+  ResidentBar* bar;
+  ResidentDir da, dt;
+};
+struct Engine;
+// Whether e's steps up to kCtlLdsJ run in one resident launch, and the launch:
+// from the state in e->dctl / e->darr until the call is done or the state
+// leaves the device phases.  e->rbar->failed is set if a barrier ran out.
+bool resident_fits(const Engine* e);
+template <typename T>
+int launch_resident(Engine* e, hipStream_t s);
+
 struct Engine {
   static constexpr unsigned kMagic = 0x504b4c42u;  // "PKLB"
   unsigned magic = 0;
@@ -267,6 +302,8 @@ struct Engine {
   hipStream_t stream = nullptr;
   int ccap = 0;                      // column capacity of one Gram-Schmidt pass: max(kMaxCols, kmax + 2)
   double* part = nullptr;            // partial sums (max_blocks * ccap)
+  size_t part_len = 0;               // doubles of part
+  ResidentBar* rbar = nullptr;       // grid barrier of the resident steps
   double* red = nullptr;             // reduced sums (ccap + 16)
   double* hred = nullptr;            // pinned host mirror of red
   int* dcols = nullptr;              // reorthogonalization column list
