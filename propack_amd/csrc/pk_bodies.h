@@ -45,58 +45,75 @@ __device__ __forceinline__ void spmv_chunk(const int4 d, const int* __restrict__
   }
 }
 
+// The row bounds, yprev and running sums of kRowPre rows of a group (rows
+// r0 + group + (it0 + u) * ngroups), loaded together ahead of their sums: one
+// memory round trip per kRowPre rows instead of two per row.  Rows past r1
+// read row r0 and are not used.
+constexpr int kRowPre = 4;
+struct RowPre {
+  int a[kRowPre], b[kRowPre];
+  double yp[kRowPre], yin[kRowPre];
+};
+template <typename T, int G, int NT>
+__device__ __forceinline__ void spmv_rows_load(RowPre& R, int it0, int r0, int r1, int p0,
+                                               const int* __restrict__ rp,
+                                               const T* __restrict__ yprev,
+                                               const double* __restrict__ yacc_in, int last) {
+  const int group = threadIdx.x / G;
+  constexpr int ngroups = NT / G;
+#pragma unroll
+  for (int u = 0; u < kRowPre; ++u) {
+    const int r = r0 + group + (it0 + u) * ngroups;
+    const int rr = r < r1 ? r : r0;
+    R.a[u] = rp[rr] - p0;
+    R.b[u] = rp[rr + 1] - p0;
+    R.yp[u] = (last && yprev) ? static_cast<double>(yprev[rr]) : 0.0;
+    R.yin[u] = yacc_in ? yacc_in[rr] : 0.0;
+  }
+}
+
 // Row sums of rows [r0, r1) from their products in LDS (prod[q] for the
 // block's q-th nonzero in row-major order): groups of G lanes, lane l of a
 // row adds prod[a + l], prod[a + l + G], ... then a shuffle tree; then the
 // epilogue.  The order depends only on G and the row, not on the block.
-template <typename T, int G, int NT>
+// PRE: R holds the first kRowPre rows' loads already.
+template <typename T, int G, int NT, bool PRE = false>
 __device__ __forceinline__ void spmv_rows(int r0, int r1, int p0, const int* __restrict__ rp,
                                           const double* prod, T* __restrict__ y,
                                           const T* __restrict__ yprev, double c, double* q_s2,
                                           double* q_sd, const double* __restrict__ yacc_in,
-                                          double* __restrict__ yacc_out, int last,
-                                          double* lds) {
+                                          double* __restrict__ yacc_out, int last, double* lds,
+                                          RowPre* pre = nullptr) {
   double s2 = 0.0, sd = 0.0;
   const int lane = threadIdx.x & (G - 1);
   const int group = threadIdx.x / G;
   constexpr int ngroups = NT / G;
   const int nrows = r1 - r0;
   const int iters = (nrows + ngroups - 1) / ngroups;  // uniform across the block
-  // The row bounds, yprev and the running sums of kPre of a group's rows
-  // are loaded together ahead of their sums (one memory round trip per kPre
-  // rows instead of two per row); loads of rows past r1 read row r0 and
-  // are not used.  The sums themselves are unchanged.
-  constexpr int kPre = 4;
-  for (int it0 = 0; it0 < iters; it0 += kPre) {
-    int a[kPre], b[kPre];
-    double yp[kPre], yin[kPre];
+  for (int it0 = 0; it0 < iters; it0 += kRowPre) {
+    RowPre R;
+    if (PRE && it0 == 0)
+      R = *pre;
+    else
+      spmv_rows_load<T, G, NT>(R, it0, r0, r1, p0, rp, yprev, yacc_in, last);
 #pragma unroll
-    for (int u = 0; u < kPre; ++u) {
-      const int r = r0 + group + (it0 + u) * ngroups;
-      const int rr = (it0 + u < iters && r < r1) ? r : r0;
-      a[u] = rp[rr] - p0;
-      b[u] = rp[rr + 1] - p0;
-      yp[u] = (last && yprev) ? static_cast<double>(yprev[rr]) : 0.0;
-      yin[u] = yacc_in ? yacc_in[rr] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < kPre; ++u) {
+    for (int u = 0; u < kRowPre; ++u) {
       if (it0 + u >= iters) break;  // uniform across the block
       const int r = r0 + group + (it0 + u) * ngroups;
       const bool valid = r < r1;
       double acc = 0.0;
       if (valid)
-        for (int q = a[u] + lane; q < b[u]; q += G) acc += prod[q];
+        for (int q = R.a[u] + lane; q < R.b[u]; q += G) acc += prod[q];
       acc = group_sum<G>(acc);
       if (valid && lane == 0) {
-        if (yacc_in) acc = yin[u] + acc;
+        if (yacc_in) acc = R.yin[u] + acc;
         if (!last) {
           yacc_out[r] = acc;
         } else {
-          const T yv = static_cast<T>(acc - c * yp[u]);
+          const T yv = static_cast<T>(acc - c * R.yp[u]);
           y[r] = yv;
           s2 += static_cast<double>(yv) * static_cast<double>(yv);
-          sd += yp[u] * static_cast<double>(yv);
+          sd += R.yp[u] * static_cast<double>(yv);
         }
       }
     }
@@ -111,8 +128,8 @@ __device__ __forceinline__ void spmv_rows(int r0, int r1, int p0, const int* __r
 }
 
 // Descriptor d = {x, y, z, w}:
-//   * y >= 0: a row block, rows [x, y) holding at most kSpmvCap nonzeros
-//     and kSpmvRows rows.  All 256 threads turn its nonzeros into products
+//   * y >= 0: a row block, rows [x, y) holding the w <= kSpmvCap nonzeros
+//     from z on and at most kSpmvRows rows.  All 256 threads turn its nonzeros into products
 //     val * x[col] in LDS (prod) -- index and value streams read fully
 //     coalesced, kUnroll independent gathers in flight per thread -- then
 //     groups of G lanes sum each row from LDS (consecutive, conflict-free
@@ -137,34 +154,38 @@ __device__ __forceinline__ void spmv_rb_body(const int4 d, const int* __restrict
     spmv_chunk<VT, T, kBlock>(d, ci, va, x, q_s2, q_sd, lsum, last, lds);
     return;
   }
-  const int r0 = d.x, r1 = d.y;
-  const int p0 = rp[r0];
-  const int nz = rp[r1] - p0;
-  // Eight independent loads per thread; with kSpmvCap = 1024 the upper
-  // half is masked, which measured faster than a 4-deep unroll.
-  constexpr int kUnroll = 8;
-  for (int base = 0; base < nz; base += kBlock * kUnroll) {
-    int idx[kUnroll];
-    double v[kUnroll], xv[kUnroll];
+  const int r0 = d.x, r1 = d.y, p0 = d.z, nz = d.w;
+  static_assert(kSpmvCap == 4 * kBlock, "four nonzeros per thread");
+  constexpr int kPer = kSpmvCap / kBlock;
+  int idx[kPer];
+  VT v[kPer];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int t = base + u * kBlock + static_cast<int>(threadIdx.x);
-      // index and value streams are read once: non-temporal, so that they
-      // do not evict the gathered vector slice from L2
-      idx[u] = t < nz ? __builtin_nontemporal_load(ci + p0 + t) : -1;
-      v[u] = t < nz ? static_cast<double>(__builtin_nontemporal_load(va + p0 + t)) : 0.0;
-    }
+  for (int u = 0; u < kPer; ++u) {
+    const int t = u * kBlock + static_cast<int>(threadIdx.x);
+    // index and value streams are read once: non-temporal, so that they
+    // do not evict the gathered vector slice from L2
+    idx[u] = t < nz ? __builtin_nontemporal_load(ci + p0 + t) : -1;
+    v[u] = t < nz ? __builtin_nontemporal_load(va + p0 + t) : VT(0);
+  }
+  // The first rows' bounds and previous values load beside the gathers: ahead
+  // of them for FP32 (200,000 x 100,000, 3.2M nonzeros: 20.9 us; behind them
+  // 22.8; after the barrier 23.0), behind them for FP64 (23.3 us; ahead 24.1;
+  // after the barrier 23.8).
+  RowPre R;
+  constexpr bool kRowsFirst = sizeof(T) == 4;
+  if (kRowsFirst) spmv_rows_load<T, G, kBlock>(R, 0, r0, r1, p0, rp, yprev, yacc_in, last);
+  T xv[kPer];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) xv[u] = idx[u] >= 0 ? static_cast<double>(x[idx[u]]) : 0.0;
+  for (int u = 0; u < kPer; ++u) xv[u] = idx[u] >= 0 ? x[idx[u]] : T(0);
+  if (!kRowsFirst) spmv_rows_load<T, G, kBlock>(R, 0, r0, r1, p0, rp, yprev, yacc_in, last);
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int t = base + u * kBlock + static_cast<int>(threadIdx.x);
-      if (t < nz) prod[t] = v[u] * xv[u];
-    }
+  for (int u = 0; u < kPer; ++u) {
+    const int t = u * kBlock + static_cast<int>(threadIdx.x);
+    if (t < nz) prod[t] = static_cast<double>(v[u]) * static_cast<double>(xv[u]);
   }
   __syncthreads();
-  spmv_rows<T, G, kBlock>(r0, r1, p0, rp, prod, y, yprev, c, q_s2, q_sd, yacc_in, yacc_out,
-                          last, lds);
+  spmv_rows<T, G, kBlock, true>(r0, r1, p0, rp, prod, y, yprev, c, q_s2, q_sd, yacc_in, yacc_out,
+                                last, lds, &R);
 }
 
 // --------------------------------------------------- row-wise SpMV ----
@@ -280,9 +301,7 @@ __device__ __forceinline__ void spmv_sorted_body(
     return;
   }
   const unsigned pmask = (1u << pbits) - 1u;
-  const int r0 = d.x, r1 = d.y;
-  const int p0 = rp[r0];
-  const int nz = rp[r1] - p0;
+  const int r0 = d.x, r1 = d.y, p0 = d.z, nz = d.w;
   constexpr int kUnroll = 8;
   for (int base = 0; base < nz; base += kSortThreads * kUnroll) {
     int idx[kUnroll], pos[kUnroll];

@@ -125,7 +125,7 @@ Partition partition(const std::vector<int>& rp, int rows, int cap = kSpmvCap,
       nz += len;
       ++r;
     }
-    P.desc.push_back(make_int4(start, r, -1, 0));
+    P.desc.push_back(make_int4(start, r, rp[start], static_cast<int>(nz)));
   }
   return P;
 }
