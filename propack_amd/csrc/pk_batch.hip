@@ -57,6 +57,7 @@ struct BPanel {
   double* lsum;
   const unsigned short* spos;
   int col0, pbits;  // packed sorted layout (CsrOp::Panel::scol0, spbits)
+  int g;            // lanes per row
 };
 
 // Work item of a batched SpMV launch: descriptor of problem pid, local
@@ -84,7 +85,47 @@ __global__ __launch_bounds__(kBlock) void k_bscale(const BProb* __restrict__ pro
 }
 
 // tr = 1: v_J = A^T u_J - beta v_{J-1}; tr = 0: u_{J+1} = A v_J - alpha u_J.
-template <typename VT, typename T, int G>
+// One launch takes the blocks of every problem in a layout, whatever its lanes
+// per row (pan.g, uniform over the workgroup): a launch per lane count ended
+// with a drain each, four of them in the batched workload (24 problems, 37M
+// nonzeros, FP32: 160 us per direction and step).
+template <typename VT, typename T>
+struct BSpmv {
+  const T* x;
+  T* y;
+  const T* yprev;
+  double c;
+  double* yin;
+  double* yout;
+  int last;
+  long long q;
+};
+template <typename VT, typename T>
+__device__ __forceinline__ BSpmv<VT, T> bspmv_args(const BProb& P, int loc, int tr, int p, int J) {
+  BSpmv<VT, T> a;
+  a.last = p == (tr ? P.npt : P.npa) - 1;
+  double* yacc = tr ? P.yacc_t : P.yacc_a;
+  a.yin = p == 0 ? nullptr : yacc;
+  a.yout = a.last ? nullptr : yacc;
+  a.x = tr ? bcol<T>(P, false, J) : bcol<T>(P, true, J);
+  a.y = tr ? bcol<T>(P, true, J) : bcol<T>(P, false, J + 1);
+  a.yprev = tr ? (J > 1 ? bcol<T>(P, true, J - 1) : nullptr) : bcol<T>(P, false, J);
+  a.c = tr ? P.ctl->beta : P.ctl->alpha;
+  a.q = (tr ? P.qt0 : P.qa0) + loc;
+  return a;
+}
+
+#define PK_LANES(g, CALL)   \
+  switch (g) {              \
+    case 2: CALL(2); break;  \
+    case 4: CALL(4); break;  \
+    case 8: CALL(8); break;  \
+    case 16: CALL(16); break; \
+    case 32: CALL(32); break; \
+    default: CALL(64); break; \
+  }
+
+template <typename VT, typename T>
 __global__ __launch_bounds__(kBlock) void k_bspmv(const BProb* __restrict__ probs,
                                                   const BPanel* __restrict__ panels,
                                                   const int4* __restrict__ desc,
@@ -97,21 +138,18 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BProb* __restrict__ prob
   __shared__ double prod[kSpmvCap];
   __shared__ double lds[(kBlock / kWave) * 2];
   const BPanel pan = panels[(w.pid * 2 + tr) * kPanelsMax + p];
-  const int np = tr ? P.npt : P.npa;
-  const int last = p == np - 1;
-  double* yacc = tr ? P.yacc_t : P.yacc_a;
-  const T* x = tr ? bcol<T>(P, false, J) : bcol<T>(P, true, J);
-  T* y = tr ? bcol<T>(P, true, J) : bcol<T>(P, false, J + 1);
-  const T* yprev = tr ? (J > 1 ? bcol<T>(P, true, J - 1) : nullptr) : bcol<T>(P, false, J);
-  const double c = tr ? P.ctl->beta : P.ctl->alpha;
-  const int q = (tr ? P.qt0 : P.qa0) + w.loc;
-  spmv_rb_body<VT, T, G>(desc[blockIdx.x], pan.rp, pan.ci, static_cast<const VT*>(pan.va), x, y,
-                         yprev, c, part + q, part + Q + q, pan.lsum, p == 0 ? nullptr : yacc,
-                         last ? nullptr : yacc, last, prod, lds);
+  const BSpmv<VT, T> a = bspmv_args<VT, T>(P, w.loc, tr, p, J);
+  const int4 d = desc[blockIdx.x];
+#define PK_CALL(G)                                                                             \
+  spmv_rb_body<VT, T, G>(d, pan.rp, pan.ci, static_cast<const VT*>(pan.va), a.x, a.y, a.yprev, \
+                         a.c, part + a.q, part + Q + a.q, pan.lsum, a.yin, a.yout, a.last, prod, \
+                         lds)
+  PK_LANES(pan.g, PK_CALL)
+#undef PK_CALL
 }
 
 // The row-wise form over the row-block descriptors (spmv_vec_body).
-template <typename VT, typename T, int G>
+template <typename VT, typename T>
 __global__ __launch_bounds__(kBlock) void k_bspmv_vec(const BProb* __restrict__ probs,
                                                       const BPanel* __restrict__ panels,
                                                       const int4* __restrict__ desc,
@@ -123,23 +161,19 @@ __global__ __launch_bounds__(kBlock) void k_bspmv_vec(const BProb* __restrict__ 
   if (Gate{P.ctl, phase, J, 0}.off()) return;
   __shared__ double lds[(kBlock / kWave) * 2];
   const BPanel pan = panels[(w.pid * 2 + tr) * kPanelsMax + p];
-  const int np = tr ? P.npt : P.npa;
-  const int last = p == np - 1;
-  double* yacc = tr ? P.yacc_t : P.yacc_a;
-  const T* x = tr ? bcol<T>(P, false, J) : bcol<T>(P, true, J);
-  T* y = tr ? bcol<T>(P, true, J) : bcol<T>(P, false, J + 1);
-  const T* yprev = tr ? (J > 1 ? bcol<T>(P, true, J - 1) : nullptr) : bcol<T>(P, false, J);
-  const double c = tr ? P.ctl->beta : P.ctl->alpha;
-  const int q = (tr ? P.qt0 : P.qa0) + w.loc;
-  spmv_vec_body<VT, T, G>(desc[blockIdx.x], pan.rp, pan.ci, static_cast<const VT*>(pan.va), x,
-                          y, yprev, c, part + q, part + Q + q, pan.lsum,
-                          p == 0 ? nullptr : yacc, last ? nullptr : yacc, last, lds);
+  const BSpmv<VT, T> a = bspmv_args<VT, T>(P, w.loc, tr, p, J);
+  const int4 d = desc[blockIdx.x];
+#define PK_CALL(G)                                                                              \
+  spmv_vec_body<VT, T, G>(d, pan.rp, pan.ci, static_cast<const VT*>(pan.va), a.x, a.y, a.yprev, \
+                          a.c, part + a.q, part + Q + a.q, pan.lsum, a.yin, a.yout, a.last, lds)
+  PK_LANES(pan.g, PK_CALL)
+#undef PK_CALL
 }
 
 // The same over the column-sorted layout (spmv_sorted_body): one
 // kSortThreads workgroup per descriptor, the launch's largest block cap of
 // dynamic LDS.
-template <typename VT, typename T, int G>
+template <typename VT, typename T>
 __global__ __launch_bounds__(kSortThreads) void k_bspmv_sorted(
     const BProb* __restrict__ probs, const BPanel* __restrict__ panels,
     const int4* __restrict__ desc, const BWork* __restrict__ work, int tr, int p, int J,
@@ -150,19 +184,14 @@ __global__ __launch_bounds__(kSortThreads) void k_bspmv_sorted(
   extern __shared__ double prod_dyn[];
   __shared__ double lds[(kSortThreads / kWave) * 2];
   const BPanel pan = panels[(w.pid * 2 + tr) * kPanelsMax + p];
-  const int np = tr ? P.npt : P.npa;
-  const int last = p == np - 1;
-  double* yacc = tr ? P.yacc_t : P.yacc_a;
-  const T* x = tr ? bcol<T>(P, false, J) : bcol<T>(P, true, J);
-  T* y = tr ? bcol<T>(P, true, J) : bcol<T>(P, false, J + 1);
-  const T* yprev = tr ? (J > 1 ? bcol<T>(P, true, J - 1) : nullptr) : bcol<T>(P, false, J);
-  const double c = tr ? P.ctl->beta : P.ctl->alpha;
-  const int q = (tr ? P.qt0 : P.qa0) + w.loc;
-  spmv_sorted_body<VT, T, G>(desc[blockIdx.x], pan.rp, pan.ci, static_cast<const VT*>(pan.va),
-                             pan.spos, pan.col0, pan.pbits, x, y, yprev, c, part + q,
-                             part + Q + q, pan.lsum,
-                             p == 0 ? nullptr : yacc, last ? nullptr : yacc, last, prod_dyn,
-                             lds);
+  const BSpmv<VT, T> a = bspmv_args<VT, T>(P, w.loc, tr, p, J);
+  const int4 d = desc[blockIdx.x];
+#define PK_CALL(G)                                                                             \
+  spmv_sorted_body<VT, T, G>(d, pan.rp, pan.ci, static_cast<const VT*>(pan.va), pan.spos,       \
+                             pan.col0, pan.pbits, a.x, a.y, a.yprev, a.c, part + a.q,          \
+                             part + Q + a.q, pan.lsum, a.yin, a.yout, a.last, prod_dyn, lds)
+  PK_LANES(pan.g, PK_CALL)
+#undef PK_CALL
 }
 
 template <typename T>
@@ -304,8 +333,8 @@ struct Batch {
   int* cslice_pid_n = nullptr;
   BPanel* panels = nullptr;    // (pid * 2 + tr) * kPanelsMax + p
   struct Launch {              // one batched SpMV launch
-    int tr, p, g, cap, count;  // cap > 0: column-sorted blocks of at most cap nonzeros;
-                               // cap < 0: row-wise over the row-block arrays
+    int tr, p, cap, count;  // cap > 0: column-sorted blocks of at most cap nonzeros;
+                            // cap < 0: row-wise over the row-block arrays
     int4* desc;
     BWork* work;
   };
@@ -357,68 +386,21 @@ void enqueue_batch_step(Batch& B, int J, int elr, int tries) {
         if (L.tr != tr || L.p != p || L.count == 0) continue;
         any = true;
         const int Q = tr ? B.Qt : B.Qa;
-#define PK_BS_CASE(G)                                                                           \
-  case G:                                                                                       \
-    if (B.val_prec == PK_F64)                                                                   \
-      hipLaunchKernelGGL((k_bspmv<double, T, G>), dim3(L.count), dim3(kBlock), 0, s, B.dprob,   \
-                         B.panels, L.desc, L.work, tr, p, J, phase, B.part, Q);                 \
-    else                                                                                        \
-      hipLaunchKernelGGL((k_bspmv<float, T, G>), dim3(L.count), dim3(kBlock), 0, s, B.dprob,    \
-                         B.panels, L.desc, L.work, tr, p, J, phase, B.part, Q);                 \
-    break;
-#define PK_BV_CASE(G)                                                                           \
-  case G:                                                                                       \
-    if (B.val_prec == PK_F64)                                                                   \
-      hipLaunchKernelGGL((k_bspmv_vec<double, T, G>), dim3(L.count), dim3(kBlock), 0, s,        \
-                         B.dprob, B.panels, L.desc, L.work, tr, p, J, phase, B.part, Q);        \
-    else                                                                                        \
-      hipLaunchKernelGGL((k_bspmv_vec<float, T, G>), dim3(L.count), dim3(kBlock), 0, s,         \
-                         B.dprob, B.panels, L.desc, L.work, tr, p, J, phase, B.part, Q);        \
-    break;
-#define PK_BSS_CASE(G)                                                                          \
-  case G:                                                                                       \
-    if (B.val_prec == PK_F64)                                                                   \
-      hipLaunchKernelGGL((k_bspmv_sorted<double, T, G>), dim3(L.count), dim3(kSortThreads), shm, \
-                         s, B.dprob, B.panels, L.desc, L.work, tr, p, J, phase, B.part, Q);     \
-    else                                                                                        \
-      hipLaunchKernelGGL((k_bspmv_sorted<float, T, G>), dim3(L.count), dim3(kSortThreads), shm,  \
-                         s, B.dprob, B.panels, L.desc, L.work, tr, p, J, phase, B.part, Q);     \
-    break;
+#define PK_BSPMV(KERNEL, NT, SHM)                                                            \
+  if (B.val_prec == PK_F64)                                                                    \
+    hipLaunchKernelGGL((KERNEL<double, T>), dim3(L.count), dim3(NT), SHM, s, B.dprob, B.panels, \
+                       L.desc, L.work, tr, p, J, phase, B.part, Q);                            \
+  else                                                                                         \
+    hipLaunchKernelGGL((KERNEL<float, T>), dim3(L.count), dim3(NT), SHM, s, B.dprob, B.panels, \
+                       L.desc, L.work, tr, p, J, phase, B.part, Q)
         if (L.cap > 0) {
-          const size_t shm = sizeof(double) * static_cast<size_t>(L.cap);
-          switch (L.g) {
-            PK_BSS_CASE(2)
-            PK_BSS_CASE(4)
-            PK_BSS_CASE(8)
-            PK_BSS_CASE(16)
-            PK_BSS_CASE(32)
-            PK_BSS_CASE(64)
-            default: break;
-          }
+          PK_BSPMV(k_bspmv_sorted, kSortThreads, sizeof(double) * static_cast<size_t>(L.cap));
         } else if (L.cap < 0) {
-          switch (L.g) {
-            PK_BV_CASE(2)
-            PK_BV_CASE(4)
-            PK_BV_CASE(8)
-            PK_BV_CASE(16)
-            PK_BV_CASE(32)
-            PK_BV_CASE(64)
-            default: break;
-          }
+          PK_BSPMV(k_bspmv_vec, kBlock, 0);
         } else {
-          switch (L.g) {
-            PK_BS_CASE(2)
-            PK_BS_CASE(4)
-            PK_BS_CASE(8)
-            PK_BS_CASE(16)
-            PK_BS_CASE(32)
-            PK_BS_CASE(64)
-            default: break;
-          }
+          PK_BSPMV(k_bspmv, kBlock, 0);
         }
-#undef PK_BS_CASE
-#undef PK_BV_CASE
-#undef PK_BSS_CASE
+#undef PK_BSPMV
       }
       for (const auto& L : B.lng) {
         if (L.tr != tr || L.p != p || L.count == 0) continue;
@@ -519,9 +501,9 @@ int batch_create(int nprob, const pk_lbd_t* handles, Batch** out) {
   int rc = PK_OK;
   std::vector<int> spm, spn, cpm, cpn;
   std::vector<BPanel> hpan(static_cast<size_t>(nprob) * 2 * kPanelsMax, BPanel{});
-  // SpMV work lists keyed by (tr, panel, lanes per row, sorted-layout cap)
+  // SpMV work lists keyed by (tr, panel, sorted-layout cap)
   struct Key {
-    int tr, p, g, cap;
+    int tr, p, cap;
     std::vector<int4> desc;
     std::vector<BWork> work;
   };
@@ -601,8 +583,9 @@ int batch_create(int nprob, const pk_lbd_t* handles, Batch** out) {
         const CsrOp::Panel& pan = D.pan[p];
         const CsrOp::Part& part = cap > 0 ? pan.spart : pan.part;
         hpan[(static_cast<size_t>(i) * 2 + tr) * kPanelsMax + p] =
-            cap > 0 ? BPanel{pan.rp, pan.sci, pan.sva, e->sw_l, pan.spos, pan.scol0, pan.spbits}
-                    : BPanel{pan.rp, pan.ci, pan.va, e->sw_l, nullptr, 0, 0};
+            cap > 0 ? BPanel{pan.rp, pan.sci, pan.sva, e->sw_l, pan.spos, pan.scol0, pan.spbits,
+                             pan.g}
+                    : BPanel{pan.rp, pan.ci, pan.va, e->sw_l, nullptr, 0, 0, pan.g};
         std::vector<int4> hd(part.ndesc), hl(part.nlong);
         if ((!hd.empty() && hipMemcpy(hd.data(), part.desc, sizeof(int4) * hd.size(),
                                       hipMemcpyDeviceToHost) != hipSuccess) ||
@@ -612,10 +595,10 @@ int batch_create(int nprob, const pk_lbd_t* handles, Batch** out) {
           break;
         }
         auto kit = std::find_if(keys.begin(), keys.end(), [&](const Key& k) {
-          return k.tr == tr && k.p == p && k.g == pan.g && k.cap == cap;
+          return k.tr == tr && k.p == p && k.cap == cap;
         });
         if (kit == keys.end()) {
-          keys.push_back(Key{tr, p, pan.g, cap, {}, {}});
+          keys.push_back(Key{tr, p, cap, {}, {}});
           kit = keys.end() - 1;
         }
         for (int b = 0; b < static_cast<int>(hd.size()); ++b) {
@@ -654,7 +637,7 @@ int batch_create(int nprob, const pk_lbd_t* handles, Batch** out) {
               upload_vec(cpm, &B->cslice_pid_m) && upload_vec(cpn, &B->cslice_pid_n) &&
               upload_vec(hpan, &B->panels);
     for (auto& k : keys) {
-      Batch::Launch L{k.tr, k.p, k.g, k.cap, static_cast<int>(k.desc.size()), nullptr, nullptr};
+      Batch::Launch L{k.tr, k.p, k.cap, static_cast<int>(k.desc.size()), nullptr, nullptr};
       ok = ok && upload_vec(k.desc, &L.desc) && upload_vec(k.work, &L.work);
       B->spmv.push_back(L);
     }
