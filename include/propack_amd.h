@@ -208,8 +208,8 @@ void pk_ccsr_aprod_(const char* transa, const int* m, const int* n, const void* 
  * is registered with pk_lbd_set_callback.  A complex prec (PK_C128 /
  * PK_C64) makes the engine of ZLANBPRO / CLANBPRO (complex16/zlanbpro.F):
  * complex bases, the same real B, its operator complex of the same
- * precision and a callback with the complex signature of that precision;
- * its steps run on the host executor.  pk_lbd_residuals, pk_lbd_promote,
+ * precision and a callback with the complex signature of that precision.
+ * pk_lbd_residuals, pk_lbd_promote,
  * pk_lbd_seed and the batched calls take real engines only.                */
 int pk_lbd_create(int prec, int m, int n, int kmax, pk_csr_t op, pk_lbd_t* eng);
 int pk_lbd_destroy(pk_lbd_t eng);

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kBlock) void k_bctl(const BProb* __restrict__ probs
   const BProb P = probs[blockIdx.x];
   __shared__ LbdCtlLds c;
   __shared__ LbdCtlRef cg;
-  __shared__ double lds[(kBlock / kWave) * 2];
+  __shared__ double lds[(kBlock / kWave) * 3];
   if (P.ctl->phase != phase || P.ctl->j != J) return;
   const double* pa;
   const double* pb = nullptr;

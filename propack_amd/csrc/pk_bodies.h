@@ -648,7 +648,8 @@ static_assert(kCtlHdrWords + 2 * kCtlWinD + kCtlWinI / 4 <= kCtlPer * kBlock,
 // The control stage itself on state c (LDS or device arrays): thread 0 runs
 // the stage, the workgroup a pending omega update, thread 0 the remainder.
 template <class C>
-__device__ __forceinline__ void ctl_run(C& c, int kind, double a, double b, double* lds) {
+__device__ __forceinline__ void ctl_run(C& c, int kind, double a, double b, double* lds,
+                                        double im = 0.0) {
   if (threadIdx.x == 0) {
     switch (kind) {
       case CTL_V_SPMV: ctl_v_spmv_s(c, a, b); break;
@@ -657,6 +658,10 @@ __device__ __forceinline__ void ctl_run(C& c, int kind, double a, double b, doub
       case CTL_U_SPMV: ctl_u_spmv_s(c, a, b); break;
       case CTL_U_ELR: ctl_u_elr_s(c, a, b); break;
       case CTL_U_REO: ctl_u_reo_s(c, a); break;
+      case CTL_ZV_SPMV: zctl_v_spmv_s(c, a, b, im); break;
+      case CTL_ZV_ELR: zctl_v_elr_s(c, a, b, im); break;
+      case CTL_ZU_SPMV: zctl_u_spmv_s(c, a, b, im); break;
+      case CTL_ZU_ELR: zctl_u_elr_s(c, a, b, im); break;
       default: break;
     }
   }
@@ -707,12 +712,13 @@ __device__ __forceinline__ void ctl_word(int w, LbdCtl* gc, char* garr, int cap,
 // loads issued before the partial reductions, reduce a = sum pa[0:na) (and
 // b = sum pb[0:nb) when pb is set) in index order, run the stage
 // (ctl_run), write the state back.  Steps past kCtlLdsJ stage the scalars
-// only and work on the arrays in device memory.  lds holds
-// (kBlock / kWave) * 2 doubles.
+// only and work on the arrays in device memory.  pc (complex stages): a third
+// array of nb partials.  lds holds (kBlock / kWave) * 3 doubles.
 __device__ __forceinline__ void ctl_stage_body(LbdCtl* __restrict__ gc, char* garr, int cap,
                                                int J, int kind, const double* pa, int na,
                                                const double* pb, int nb, LbdCtlLds& c,
-                                               LbdCtlRef& cg, double* lds) {
+                                               LbdCtlRef& cg, double* lds,
+                                               const double* pc = nullptr) {
   const bool in_lds = J <= kCtlLdsJ;
   const int wd = (J + 4) & ~1, wi = (2 * J + 8) & ~3;
   const int nw = in_lds ? kCtlHdrWords + 2 * wd + wi / 4 : kCtlHdrWords;
@@ -731,8 +737,15 @@ __device__ __forceinline__ void ctl_stage_body(LbdCtl* __restrict__ gc, char* ga
   ctl_word(min(t + 4 * kBlock, nw - 1), gc, garr, cap, wd, c, &s4, &d4);
   ctl_word(min(t + 5 * kBlock, nw - 1), gc, garr, cap, wd, c, &s5, &d5);
   const int4 w0 = *s0, w1 = *s1, w2 = *s2, w3 = *s3, w4 = *s4, w5 = *s5;
-  double a, b = 0.0;
-  if (pb && nb == na) {
+  double a, b = 0.0, im = 0.0;
+  if (pc) {
+    const double* const q[3] = {pa, pb, pc};
+    double v[3];
+    reduce_partials_n<3>(q, na, v, lds);
+    a = v[0];
+    b = v[1];
+    im = v[2];
+  } else if (pb && nb == na) {
     const double* const q[2] = {pa, pb};
     double v[2];
     reduce_partials_n<2>(q, na, v, lds);
@@ -751,14 +764,14 @@ __device__ __forceinline__ void ctl_stage_body(LbdCtl* __restrict__ gc, char* ga
   __syncthreads();
   if (in_lds) {
     if (threadIdx.x == 0) c.cols = CtlArrays::cols(garr, cap);
-    ctl_run(c, kind, a, b, lds);
+    ctl_run(c, kind, a, b, lds, im);
   } else {
     if (threadIdx.x == 0) {
       *static_cast<LbdCtl*>(&cg) = *static_cast<LbdCtl*>(&c);
       cg.bind(garr);
     }
     __syncthreads();
-    ctl_run(cg, kind, a, b, lds);
+    ctl_run(cg, kind, a, b, lds, im);
     if (threadIdx.x == 0) *static_cast<LbdCtl*>(&c) = *static_cast<LbdCtl*>(&cg);
     __syncthreads();
   }

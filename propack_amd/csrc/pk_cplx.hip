@@ -68,8 +68,11 @@ __global__ __launch_bounds__(kBlock) void k_zspmv(long long rows, const int* __r
                                                   const typename V2T<R>::type* __restrict__ x,
                                                   typename V2T<R>::type* __restrict__ y,
                                                   const typename V2T<R>::type* __restrict__ yprev,
-                                                  double c, double* __restrict__ part) {
+                                                  Scal coef, double* __restrict__ part,
+                                                  Gate gate) {
   using C2 = typename V2T<R>::type;
+  if (gate.off()) return;
+  const double c = coef.get();
   __shared__ double lds[(kBlock / kWave) * 3];
   constexpr int ngrp = kBlock / G;
   const int lane = threadIdx.x % G, grp = threadIdx.x / G;
@@ -144,8 +147,9 @@ template <typename R, int G>
 __global__ __launch_bounds__(kBlock) void k_zspmv_cp(long long rows, int np, ZPanels tab,
                                                      int conj,
                                                      const typename V2T<R>::type* __restrict__ x,
-                                                     double2* __restrict__ ypart) {
+                                                     double2* __restrict__ ypart, Gate gate) {
   using C2 = typename V2T<R>::type;
+  if (gate.off()) return;
   constexpr int ngrp = kBlock / G;
   const int lane = threadIdx.x % G, grp = threadIdx.x / G;
   const int pn = static_cast<int>(blockIdx.x % np);
@@ -195,10 +199,12 @@ template <typename R, int NP>
 __global__ __launch_bounds__(kBlock) void k_zcombine(long long rows, int np,
                                                      const double2* __restrict__ ypart,
                                                      const typename V2T<R>::type* __restrict__ yprev,
-                                                     double c,
+                                                     Scal coef,
                                                      typename V2T<R>::type* __restrict__ y,
-                                                     double* __restrict__ part) {
+                                                     double* __restrict__ part, Gate gate) {
   using C2 = typename V2T<R>::type;
+  if (gate.off()) return;
+  const double c = coef.get();
   __shared__ double lds[(kBlock / kWave) * 3];
   const long long base = static_cast<long long>(blockIdx.x) * kZRows + threadIdx.x;
   double acc[3] = {0.0, 0.0, 0.0};
@@ -269,9 +275,12 @@ template <typename R>
 __global__ __launch_bounds__(kBlock) void k_zaxpy_norm_dot(long long L,
                                                            typename V2T<R>::type* __restrict__ w,
                                                            const typename V2T<R>::type* __restrict__ v,
-                                                           double sr, double si,
-                                                           double* __restrict__ part) {
+                                                           Scal s_re, Scal s_im,
+                                                           double* __restrict__ part,
+                                                           Gate gate) {
   using C2 = typename V2T<R>::type;
+  if (gate.off()) return;
+  const double sr = s_re.get(), si = s_im.get();
   __shared__ double lds[(kBlock / kWave) * 3];
   const long long base = static_cast<long long>(blockIdx.x) * kZRows + threadIdx.x;
   double acc[3] = {0.0, 0.0, 0.0};
@@ -311,10 +320,12 @@ template <typename R>
 __global__ __launch_bounds__(kBlock) void k_zgemvt(long long L,
                                                    const typename V2T<R>::type* __restrict__ V,
                                                    long long ldv, const int* __restrict__ cols,
-                                                   int ncols,
+                                                   int ncols_v, const int* ncols_p,
                                                    const typename V2T<R>::type* __restrict__ w,
-                                                   double* __restrict__ part) {
+                                                   double* __restrict__ part, Gate gate) {
   using C2 = typename V2T<R>::type;
+  if (gate.off()) return;
+  const int ncols = ncols_p ? *ncols_p : ncols_v;
   __shared__ double lds[(kBlock / kWave) * 2 * kZCols];
   const size_t nb = gridDim.x;
   if (L <= 0) {  // empty vectors: zero projections, no loads
@@ -373,11 +384,14 @@ template <typename R>
 __global__ __launch_bounds__(kBlock) void k_zgemv_update(long long L,
                                                          const typename V2T<R>::type* __restrict__ V,
                                                          long long ldv,
-                                                         const int* __restrict__ cols, int ncols,
+                                                         const int* __restrict__ cols,
+                                                         int ncols_v, const int* ncols_p,
                                                          const double* __restrict__ h,
                                                          typename V2T<R>::type* __restrict__ w,
-                                                         double* __restrict__ part) {
+                                                         double* __restrict__ part, Gate gate) {
   using C2 = typename V2T<R>::type;
+  if (gate.off()) return;
+  const int ncols = ncols_p ? *ncols_p : ncols_v;
   __shared__ double lds[kBlock / kWave];
   if (L <= 0) {
     if (threadIdx.x == 0) part[blockIdx.x] = 0.0;
@@ -455,14 +469,14 @@ int zspmv_lanes(long long nnz, long long rows) {
 
 template <typename R>
 int launch_zspmv(hipStream_t s, long long rows, const int* rp, const int* ci, const void* va,
-                 int conj, int g, const void* x, void* y, const void* yprev, double c,
-                 double* part) {
+                 int conj, int g, const void* x, void* y, const void* yprev, Scal c,
+                 double* part, Gate gate) {
   using C2 = typename V2T<R>::type;
   const int nblk = zspmv_blocks(rows, g);
 #define PK_ZSPMV(G)                                                                            \
   hipLaunchKernelGGL((k_zspmv<R, G>), dim3(nblk), dim3(kBlock), 0, s, rows, rp, ci,             \
                      static_cast<const C2*>(va), conj, static_cast<const C2*>(x),               \
-                     static_cast<C2*>(y), static_cast<const C2*>(yprev), c, part)
+                     static_cast<C2*>(y), static_cast<const C2*>(yprev), c, part, gate)
   switch (g) {
     case 2: PK_ZSPMV(2); break;
     case 4: PK_ZSPMV(4); break;
@@ -476,32 +490,34 @@ int launch_zspmv(hipStream_t s, long long rows, const int* rp, const int* ci, co
 }
 
 template <typename R>
-int launch_zaxpy_norm_dot(hipStream_t s, long long L, void* w, const void* v, double sr,
-                          double si, double* part) {
+int launch_zaxpy_norm_dot(hipStream_t s, long long L, void* w, const void* v, Scal sr, Scal si,
+                          double* part, Gate gate) {
   using C2 = typename V2T<R>::type;
   const int nblk = zstream_blocks(L);
   hipLaunchKernelGGL(k_zaxpy_norm_dot<R>, dim3(nblk), dim3(kBlock), 0, s, L, static_cast<C2*>(w),
-                     static_cast<const C2*>(v), sr, si, part);
+                     static_cast<const C2*>(v), sr, si, part, gate);
   return hipGetLastError() == hipSuccess ? nblk : -1;
 }
 
 template <typename R>
 int launch_zgemvt(hipStream_t s, long long L, const void* V, long long ldv, const int* cols,
-                  int ncols, const void* w, double* part) {
+                  int ncols, const int* ncols_p, const void* w, double* part, Gate gate) {
   using C2 = typename V2T<R>::type;
   const int nblk = zstream_blocks(L);
   hipLaunchKernelGGL(k_zgemvt<R>, dim3(nblk), dim3(kBlock), 0, s, L, static_cast<const C2*>(V),
-                     ldv, cols, ncols, static_cast<const C2*>(w), part);
+                     ldv, cols, ncols, ncols_p, static_cast<const C2*>(w), part, gate);
   return hipGetLastError() == hipSuccess ? nblk : -1;
 }
 
 template <typename R>
 int launch_zgemv_update(hipStream_t s, long long L, const void* V, long long ldv,
-                        const int* cols, int ncols, const double* h, void* w, double* part) {
+                        const int* cols, int ncols, const int* ncols_p, const double* h, void* w,
+                        double* part, Gate gate) {
   using C2 = typename V2T<R>::type;
   const int nblk = zstream_blocks(L);
   hipLaunchKernelGGL(k_zgemv_update<R>, dim3(nblk), dim3(kBlock), 0, s, L,
-                     static_cast<const C2*>(V), ldv, cols, ncols, h, static_cast<C2*>(w), part);
+                     static_cast<const C2*>(V), ldv, cols, ncols, ncols_p, h, static_cast<C2*>(w), part,
+                     gate);
   return hipGetLastError() == hipSuccess ? nblk : -1;
 }
 
@@ -514,7 +530,8 @@ long long zcsr_ywork(const CsrOp* op) {
 
 template <typename R>
 static int launch_zspmv_cp(hipStream_t s, const CsrOp::Dir& D, int conj, const void* x,
-                           void* y, const void* yprev, double c, double* part, double* ywork) {
+                           void* y, const void* yprev, Scal c, double* part, double* ywork,
+                           Gate gate) {
   using C2 = typename V2T<R>::type;
   ZPanels tab{};
   for (int p = 0; p < D.np; ++p) {
@@ -531,7 +548,7 @@ static int launch_zspmv_cp(hipStream_t s, const CsrOp::Dir& D, int conj, const v
   double2* yp = reinterpret_cast<double2*>(ywork);
 #define PK_ZSPMV_CP(G)                                                                       \
   hipLaunchKernelGGL((k_zspmv_cp<R, G>), dim3(grid), dim3(kBlock), 0, s, rows, np, tab, conj, \
-                     static_cast<const C2*>(x), yp)
+                     static_cast<const C2*>(x), yp, gate)
   switch (g) {
     case 2: PK_ZSPMV_CP(2); break;
     case 4: PK_ZSPMV_CP(4); break;
@@ -545,7 +562,7 @@ static int launch_zspmv_cp(hipStream_t s, const CsrOp::Dir& D, int conj, const v
   const int nblk = zstream_blocks(rows);
 #define PK_ZCB(NP)                                                                         \
   hipLaunchKernelGGL((k_zcombine<R, NP>), dim3(nblk), dim3(kBlock), 0, s, rows, np, yp,      \
-                     static_cast<const C2*>(yprev), c, static_cast<C2*>(y), part)
+                     static_cast<const C2*>(yprev), c, static_cast<C2*>(y), part, gate)
   switch (np) {
     case 2: PK_ZCB(2); break;
     case 4: PK_ZCB(4); break;
@@ -560,29 +577,29 @@ static int launch_zspmv_cp(hipStream_t s, const CsrOp::Dir& D, int conj, const v
 // 'c': A^H); returns the partial-slot count (three values per slot).
 template <typename R>
 int zcsr_apply(const CsrOp* op, hipStream_t s, char trans, const void* x, void* y,
-               const void* yprev, double c, double* part, double* ywork) {
+               const void* yprev, Scal c, double* part, double* ywork, Gate gate) {
   const bool tr = trans != 'n' && trans != 'N';
   const bool cj = trans == 'c' || trans == 'C';
   const CsrOp::Dir& D = tr ? op->dt : op->da;
   if (D.np > 1) {
     if (!ywork) return -1;
-    return launch_zspmv_cp<R>(s, D, cj ? 1 : 0, x, y, yprev, c, part, ywork);
+    return launch_zspmv_cp<R>(s, D, cj ? 1 : 0, x, y, yprev, c, part, ywork, gate);
   }
   const CsrOp::Panel& P = D.pan[0];
-  return launch_zspmv<R>(s, D.rows, P.rp, P.ci, P.va, cj ? 1 : 0, P.g, x, y, yprev, c, part);
+  return launch_zspmv<R>(s, D.rows, P.rp, P.ci, P.va, cj ? 1 : 0, P.g, x, y, yprev, c, part,
+                         gate);
 }
 
 #define PK_INST_Z(R)                                                                            \
-  template int launch_zspmv<R>(hipStream_t, long long, const int*, const int*, const void*, int, \
-                               int, const void*, void*, const void*, double, double*);          \
-  template int launch_zaxpy_norm_dot<R>(hipStream_t, long long, void*, const void*, double,     \
-                                        double, double*);                                       \
+  template int launch_zaxpy_norm_dot<R>(hipStream_t, long long, void*, const void*, Scal, Scal,  \
+                                        double*, Gate);                                         \
   template int launch_zgemvt<R>(hipStream_t, long long, const void*, long long, const int*, int, \
-                                const void*, double*);                                          \
+                                const int*, const void*, double*, Gate);                        \
   template int launch_zgemv_update<R>(hipStream_t, long long, const void*, long long,           \
-                                      const int*, int, const double*, void*, double*);          \
+                                      const int*, int, const int*, const double*, void*,        \
+                                      double*, Gate);                                           \
   template int zcsr_apply<R>(const CsrOp*, hipStream_t, char, const void*, void*, const void*,  \
-                             double, double*, double*);
+                             Scal, double*, double*, Gate);
 PK_INST_Z(double)
 PK_INST_Z(float)
 #undef PK_INST_Z

@@ -981,8 +981,8 @@ int zspmv_any(CsrOp* op, char trans, const void* x, void* y, int where) {
   }
   if (rc == PK_OK) {
     const int nb = op->val_prec == PK_C128
-                       ? zcsr_apply<double>(op, s, trans, dx, dy, nullptr, 0.0, part, yw)
-                       : zcsr_apply<float>(op, s, trans, dx, dy, nullptr, 0.0, part, yw);
+                       ? zcsr_apply<double>(op, s, trans, dx, dy, nullptr, sval(0.0), part, yw)
+                       : zcsr_apply<float>(op, s, trans, dx, dy, nullptr, sval(0.0), part, yw);
     if (nb < 0) rc = PK_ERR_HIP;
   }
   if (rc == PK_OK && where == PK_HOST &&

@@ -438,9 +438,6 @@ struct Impl {
     return PK_OK;
   }
 
-  // Execute the current phase of the step on the host (lbd_host_phase).
-  int host_phase(LbdCtlRef& c) { return lbd_host_phase(*this, c); }
-
   int zero(T* x, long long L) {
     PK_LAUNCH(launch_fill_zero_bytes(strm, x, sizeof(T) * L));
     return PK_OK;
@@ -560,7 +557,8 @@ struct Impl {
 
   // Run steps c.j..c.k on the device until done or until the state needs
   // the host (a rare path, or more CGS passes than the chain holds).
-  int run_device(LbdCtlRef& c, int elr) {
+  int run_device(LbdCtlRef& c) {
+    const int elr = c.elr;
     const long long pv0 = c.npass_v, pu0 = c.npass_u, cv0 = c.ncols_v, cu0 = c.ncols_u;
     const size_t ab = static_cast<size_t>(CtlArrays::bytes(e->kmax));
     PK_HIP(hipMemcpyAsync(e->dctl, static_cast<LbdCtl*>(&c), sizeof(LbdCtl),
@@ -617,28 +615,8 @@ struct Impl {
     return lbd_begin(*this, k0, k_in, alpha_, beta_, rnorm, doption, ioption, ierr_out, finished);
   }
 
-  // Steps of the call from the state in e->hctl until it is done: device
-  // chains from PH_V_SPMV, host execution of every other phase.
-  int lanbpro_loop() {
-    LbdCtlRef& c = *e->hctl;
-    const bool device = e->mode == 0 && e->op != nullptr;
-    while (c.phase != PH_DONE) {
-      if (device && c.phase == PH_V_SPMV) {
-        const int j_before = c.j;
-        PK_TRY(run_device(c, c.elr));
-        // A chain always advances at least one phase; if it did not, finish
-        // the step on the host rather than enqueue the same chain again.
-        if (c.phase != PH_V_SPMV || c.j != j_before) continue;
-      }
-      // a chain that stopped in a CGS phase ran out of passes: hold two
-      // passes in the engine's later chains
-      if (device && e->tries_auto && e->dev_tries < 2 &&
-          (c.phase == PH_V_REO || c.phase == PH_U_REO))
-        e->dev_tries = 2;
-      PK_TRY(host_phase(c));
-    }
-    return PK_OK;
-  }
+  // Steps of the call from the state in e->hctl until it is done (lbd_loop).
+  int lanbpro_loop() { return lbd_loop(*this, e->mode == 0 && e->op != nullptr); }
 
   // End of the call (lbd_end).
   int lanbpro_end(int k0, int* kp, double* alpha_, double* beta_, double* rnorm, double* doption,
@@ -697,39 +675,6 @@ struct Impl {
 };
 
 // ---- complex bases: ZLANBPRO / CLANBPRO ----
-// Extended local reorthogonalization of the complex tree
-// (complex16/zlanbpro.F:316-335 for v, :449-466 for u): the coefficient
-// s = v_{j-1}^H v_j is complex, so B keeps its entry (the real tree adds s
-// to it); otherwise the stage is the real one.  nsd is the real part of the
-// next coefficient.
-static void zctl_v_elr(LbdCtlRef& c, double ns2, double nsd) {
-  const double sn = std::sqrt(ns2);
-  c.elr_i++;
-  if (sn >= c.kappa * c.alpha || c.elr_i >= c.elr) {
-    c.nu[c.j - 1] = c.eps;
-    c.alpha = sn;
-    ctl_v_fin(c);
-  } else {
-    c.alpha = sn;
-    c.elr_s = nsd;
-  }
-  ctl_resume(c);
-}
-
-static void zctl_u_elr(LbdCtlRef& c, double ns2, double nsd) {
-  const double sn = std::sqrt(ns2);
-  c.elr_i++;
-  if (sn >= c.kappa * c.beta || c.elr_i >= c.elr) {
-    c.mu[c.j] = c.eps;
-    c.beta = sn;
-    ctl_u_fin(c);
-  } else {
-    c.beta = sn;
-    c.elr_s = nsd;
-  }
-  ctl_resume(c);
-}
-
 template <typename R>
 struct CxOf;
 template <>
@@ -742,11 +687,11 @@ struct CxOf<float> {
 };
 
 // The engine over complex bases (PK_C128: R = double, PK_C64: R = float).
-// Every step runs on the host executor (the phase machine of pk_lbd.h), one
-// synchronization per reduction; norms, real scalings, the random start
-// vector and the GEMMs run the real kernels on the 2L-long real view of a
-// column, the operator, dot products and Gram-Schmidt the complex kernels
-// of pk_cplx.hip.
+// Norms, real scalings, the random start vector and the GEMMs run the real
+// kernels on the 2L-long real view of a column, the operator, dot products
+// and Gram-Schmidt the complex kernels of pk_cplx.hip; the steps run as the
+// real engine's gated chains (class timing runs them on the host executor,
+// which launches only what a step needs).
 template <typename R>
 struct ZImpl {
   using Real = R;
@@ -825,7 +770,8 @@ struct ZImpl {
                            (rows_out + 1) * 4.0 + rows_in * sb + rows_out * sb +
                            (yprev ? rows_out * sb : 0.0);
       hipEvent_t t0 = tstart(tr ? KC_SPMV_T : KC_SPMV_N);
-      nb = zcsr_apply<R>(e->op, strm, tr ? 'c' : 'n', x, y, yprev, c, e->part, e->sw_y);
+      nb = zcsr_apply<R>(e->op, strm, tr ? 'c' : 'n', x, y, yprev, sval(c), e->part,
+                         e->sw_y);
       PK_LAUNCH(nb);
       tstop(t0, tr ? KC_SPMV_T : KC_SPMV_N, bytes, 8.0 * nnz);
     } else if (e->aprod) {
@@ -837,7 +783,7 @@ struct ZImpl {
         *sdr = *sdi = 0.0;
         return PK_OK;
       }
-      nb = launch_zaxpy_norm_dot<R>(strm, rows_out, y, yprev, c, 0.0, e->part);
+      nb = launch_zaxpy_norm_dot<R>(strm, rows_out, y, yprev, sval(c), sval(0.0), e->part);
       PK_LAUNCH(nb);
     } else {
       set_error("engine has no operator");
@@ -871,13 +817,13 @@ struct ZImpl {
   int cgs_pass(long long L, const T* basis, long long ld, T* vnew, int ncols, double* s2) {
     const double sb = static_cast<double>(sizeof(T));
     hipEvent_t t0 = tstart(KC_GEMVT);
-    const int nb = launch_zgemvt<R>(strm, L, basis, ld, e->dcols, ncols, vnew, e->part);
+    const int nb = launch_zgemvt<R>(strm, L, basis, ld, e->dcols, ncols, nullptr, vnew, e->part);
     PK_LAUNCH(nb);
     tstop(t0, KC_GEMVT, (ncols + 1.0) * L * sb, 8.0 * ncols * L);
     PK_LAUNCH(launch_reduce(strm, 2 * ncols, nb, e->part, e->red, Gate{}));
     hipEvent_t t1 = tstart(KC_GEMV);
-    const int nb2 = launch_zgemv_update<R>(strm, L, basis, ld, e->dcols, ncols, e->red, vnew,
-                                           e->part);
+    const int nb2 = launch_zgemv_update<R>(strm, L, basis, ld, e->dcols, ncols, nullptr, e->red,
+                                           vnew, e->part);
     PK_LAUNCH(nb2);
     tstop(t1, KC_GEMV, (ncols + 2.0) * L * sb, 8.0 * ncols * L);
     PK_LAUNCH(launch_reduce(strm, 1, nb2, e->part, hsum(), Gate{}));
@@ -990,16 +936,14 @@ struct ZImpl {
       }
       PK_TRY(apply('c', ucol(j), vcol(j), j > 1 ? vcol(j - 1) : nullptr, j > 1 ? c.beta : 0.0,
                    &s2, &sr, &si));
-      e->elr_im = si;
-      ctl_v_spmv(c, s2, sr);
+      zctl_v_spmv(c, s2, sr, si);
     } else {
       if (c.vscale) {
         PK_TRY(scale(vcol(j), e->n, c.vscale_f));
         c.vscale = 0;
       }
       PK_TRY(apply('n', vcol(j), ucol(j + 1), ucol(j), c.alpha, &s2, &sr, &si));
-      e->elr_im = si;
-      ctl_u_spmv(c, s2, sr);
+      zctl_u_spmv(c, s2, sr, si);
     }
     return PK_OK;
   }
@@ -1011,27 +955,87 @@ struct ZImpl {
     const long long L = vside ? e->n : e->m;
     T* w = vside ? vcol(j) : ucol(j + 1);
     const T* v = vside ? vcol(j - 1) : ucol(j);
-    const int nb = launch_zaxpy_norm_dot<R>(strm, L, w, v, c.elr_s, e->elr_im, e->part);
+    const int nb = launch_zaxpy_norm_dot<R>(strm, L, w, v, sval(c.elr_s), sval(c.elr_im), e->part);
     PK_LAUNCH(nb);
     PK_LAUNCH(launch_reduce(strm, 3, nb, e->part, e->red, Gate{}));
     PK_TRY(read(0, 3));
-    e->elr_im = e->hred[2];
     if (vside)
-      zctl_v_elr(c, e->hred[0], e->hred[1]);
+      zctl_v_elr(c, e->hred[0], e->hred[1], e->hred[2]);
     else
-      zctl_u_elr(c, e->hred[0], e->hred[1]);
+      zctl_u_elr(c, e->hred[0], e->hred[1], e->hred[2]);
     return PK_OK;
   }
 
-  // zlanbpro (complex16/zlanbpro.F:1-553): every phase on the host executor.
+  // One side's chain of step J: the pending scaling of x, the operator, the
+  // ELR updates, the CGS passes, each gated on the control state.
+  int enqueue_side(int J, bool vside, int elr, int tries) {
+    LbdCtl* dc = e->dctl;
+    const int* dcl = CtlArrays::cols(e->darr, e->kmax);
+    const long long L = vside ? e->n : e->m, lx = vside ? e->m : e->n;
+    T* x = vside ? ucol(J) : vcol(J);
+    T* w = vside ? vcol(J) : ucol(J + 1);
+    const T* wprev = vside ? (J > 1 ? vcol(J - 1) : nullptr) : ucol(J);
+    const T* basis = vside ? V() : U();
+    const long long ld = vside ? e->ldv : e->ldu;
+    const int p_spmv = vside ? PH_V_SPMV : PH_U_SPMV, p_elr = vside ? PH_V_ELR : PH_U_ELR,
+              p_reo = vside ? PH_V_REO : PH_U_REO;
+    PK_LAUNCH(launch_scale<R>(strm, 2 * lx, re(x), sptr(vside ? &dc->uscale_f : &dc->vscale_f),
+                              Gate{dc, p_spmv, J, vside ? 2 : 1}));
+    int nb = zcsr_apply<R>(e->op, strm, vside ? 'c' : 'n', x, w, wprev,
+                           sptr(vside ? &dc->beta : &dc->alpha), e->part, e->sw_y,
+                           Gate{dc, p_spmv, J, 0});
+    PK_LAUNCH(nb);
+    PK_LAUNCH(launch_ctl(strm, dc, e->darr, e->kmax, vside ? CTL_ZV_SPMV : CTL_ZU_SPMV, p_spmv, J,
+                         e->part, nb));
+    const int ncols = vside ? J - 1 : J;
+    if (ncols < 1) return PK_OK;
+    for (int i = 0; i < elr; ++i) {
+      nb = launch_zaxpy_norm_dot<R>(strm, L, w, wprev, sptr(&dc->elr_s), sptr(&dc->elr_im),
+                                    e->part, Gate{dc, p_elr, J, 0});
+      PK_LAUNCH(nb);
+      PK_LAUNCH(launch_ctl(strm, dc, e->darr, e->kmax, vside ? CTL_ZV_ELR : CTL_ZU_ELR, p_elr, J,
+                           e->part, nb));
+    }
+    for (int t = 0; t < tries; ++t) {
+      const Gate g{dc, p_reo, J, 0};
+      nb = launch_zgemvt<R>(strm, L, basis, ld, dcl, ncols, &dc->reo_ncols, w, e->part, g);
+      PK_LAUNCH(nb);
+      PK_LAUNCH(launch_reduce(strm, 2 * ncols, nb, e->part, e->red, g, &dc->reo_ncols, 2));
+      nb = launch_zgemv_update<R>(strm, L, basis, ld, dcl, ncols, &dc->reo_ncols, e->red, w,
+                                  e->part, g);
+      PK_LAUNCH(nb);
+      PK_LAUNCH(launch_ctl(strm, dc, e->darr, e->kmax, vside ? CTL_V_REO : CTL_U_REO, p_reo, J,
+                           e->part, nb));
+    }
+    return PK_OK;
+  }
+
+  // Run steps c.j..c.k on the device (as Impl::run_device).
+  int run_device(LbdCtlRef& c) {
+    const size_t ab = static_cast<size_t>(CtlArrays::bytes(e->kmax));
+    PK_HIP(hipMemcpyAsync(e->dctl, static_cast<LbdCtl*>(&c), sizeof(LbdCtl),
+                          hipMemcpyHostToDevice, strm));
+    PK_HIP(hipMemcpyAsync(e->darr, e->harr, ab, hipMemcpyHostToDevice, strm));
+    for (int J = c.j; J <= c.k; ++J) {
+      PK_TRY(enqueue_side(J, true, c.elr, e->dev_tries));
+      PK_TRY(enqueue_side(J, false, c.elr, e->dev_tries));
+    }
+    PK_HIP(hipMemcpyAsync(static_cast<LbdCtl*>(&c), e->dctl, sizeof(LbdCtl),
+                          hipMemcpyDeviceToHost, strm));
+    PK_HIP(hipMemcpyAsync(e->harr, e->darr, ab, hipMemcpyDeviceToHost, strm));
+    PK_HIP(stream_wait(strm));
+    e->cnt.nsync++;
+    return resolve_timers();
+  }
+
+  // zlanbpro (complex16/zlanbpro.F:1-553).
   int lanbpro(int k0, int* kp, double* alpha_, double* beta_, double* rnorm, double* doption,
               const int* ioption, int* ierr_out) {
     bool finished = false;
     PK_TRY(lbd_begin(*this, k0, *kp, alpha_, beta_, rnorm, doption, ioption, ierr_out,
                      &finished));
     if (finished) return PK_OK;
-    LbdCtlRef& c = *e->hctl;
-    while (c.phase != PH_DONE) PK_TRY(lbd_host_phase(*this, c));
+    PK_TRY(lbd_loop(*this, e->mode == 0 && e->op != nullptr && !e->prof.on));
     return lbd_end(*this, k0, kp, alpha_, beta_, rnorm, doption, ierr_out);
   }
 

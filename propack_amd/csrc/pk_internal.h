@@ -198,21 +198,22 @@ int zspmv_blocks(long long rows, int g);  // <= kMaxBlocks
 // zcsr_ywork(op) doubles (the panels' FP64 row sums).
 template <typename R>
 int zcsr_apply(const CsrOp* op, hipStream_t s, char trans, const void* x, void* y,
-               const void* yprev, double c, double* part, double* ywork);
+               const void* yprev, Scal c, double* part, double* ywork, Gate gate = Gate{});
 long long zcsr_ywork(const CsrOp* op);
 // w -= s v (complex s = sr + i si); partials ||w||^2, Re and Im of v^H w.
 template <typename R>
-int launch_zaxpy_norm_dot(hipStream_t s, long long L, void* w, const void* v, double sr,
-                          double si, double* part);
+int launch_zaxpy_norm_dot(hipStream_t s, long long L, void* w, const void* v, Scal sr, Scal si,
+                          double* part, Gate gate = Gate{});
 // Partials of h = V(:, cols)^H w: real and imaginary parts of h_j at
 // part[(2j) * nblk + b] and part[(2j+1) * nblk + b].
 template <typename R>
 int launch_zgemvt(hipStream_t s, long long L, const void* V, long long ldv, const int* cols,
-                  int ncols, const void* w, double* part);
+                  int ncols, const int* ncols_p, const void* w, double* part, Gate gate = Gate{});
 // w -= V(:, cols) h (h as 2 ncols doubles, re / im pairs); partial ||w||^2.
 template <typename R>
 int launch_zgemv_update(hipStream_t s, long long L, const void* V, long long ldv,
-                        const int* cols, int ncols, const double* h, void* w, double* part);
+                        const int* cols, int ncols, const int* ncols_p, const double* h, void* w,
+                        double* part, Gate gate = Gate{});
 
 // Fortran APROD callback: (TRANSA, M, N, X, Y, DPARM, IPARM, len(TRANSA)).
 typedef void (*aprod_d_fn)(const char*, const int*, const int*, const double*, double*,
@@ -332,9 +333,6 @@ struct Engine {
   // accumulation, where max(m, n) * 2^-24 would exceed the Lanczos residuals
   // of large problems and flag false invariant subspaces).
   int rounding = 0;
-  // complex bases (prec PK_C128 / PK_C64): the imaginary part of the
-  // pending ELR coefficient (its real part is LbdCtl::elr_s)
-  double elr_im = 0.0;
   Counters cnt;
   Profile prof;
   int last_error = 0;

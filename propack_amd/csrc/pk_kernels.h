@@ -75,9 +75,10 @@ template <typename T>
 int launch_spmv_combine(hipStream_t s, long long rows, int np, const double* ypart,
                         const T* yprev, Scal coef, T* y, double* part, Gate gate);
 
-// part (nval x nblk) -> out[v] = sum_b part[v*nblk+b] in index order.
+// part (nval x nblk) -> out[v] = sum_b part[v*nblk+b] in index order; of the
+// nval values the first *nval_p * per when nval_p is set.
 int launch_reduce(hipStream_t s, int nval, int nblk, const double* part, double* out,
-                  Gate gate, const int* nval_p = nullptr);
+                  Gate gate, const int* nval_p = nullptr, int per = 1);
 
 // h_part(ncols x nblk) = partial V(:,cols)^T w over row blocks
 // (nblk = cgs_blocks(L), returned).
@@ -147,7 +148,11 @@ int launch_gemm_group(hipStream_t s, const GemmJob* jobs, int njobs, GemmItem** 
                       size_t* dcap);
 
 // Control kernel of the device-resident step (see pk_lbd.h).
-enum CtlKind { CTL_V_SPMV = 0, CTL_V_ELR, CTL_V_REO, CTL_U_SPMV, CTL_U_ELR, CTL_U_REO };
+// (complex bases: three partials per slot for the operator and ELR stages).
+enum CtlKind {
+  CTL_V_SPMV = 0, CTL_V_ELR, CTL_V_REO, CTL_U_SPMV, CTL_U_ELR, CTL_U_REO,
+  CTL_ZV_SPMV, CTL_ZV_ELR, CTL_ZU_SPMV, CTL_ZU_ELR
+};
 int launch_ctl(hipStream_t s, LbdCtl* c, void* arrays, int cap, int kind, int want_phase,
                int want_j, const double* part, int nb);
 

@@ -307,18 +307,18 @@ int launch_spmv_combine(hipStream_t s, long long rows, int np, const double* ypa
 // -------------------------------------------------------------- reduce ----
 __global__ __launch_bounds__(kBlock) void k_reduce(int nblk, const double* __restrict__ part,
                                                    double* __restrict__ out,
-                                                   const int* nval_p, Gate gate) {
+                                                   const int* nval_p, int per, Gate gate) {
   if (gate.off()) return;
-  if (nval_p && static_cast<int>(blockIdx.x) >= *nval_p) return;
+  if (nval_p && static_cast<int>(blockIdx.x) >= *nval_p * per) return;
   __shared__ double lds[kBlock / kWave];
   const double v = reduce_partials(part + static_cast<size_t>(blockIdx.x) * nblk, nblk, lds);
   if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
 int launch_reduce(hipStream_t s, int nval, int nblk, const double* part, double* out,
-                  Gate gate, const int* nval_p) {
+                  Gate gate, const int* nval_p, int per) {
   if (nval <= 0) return 0;
-  hipLaunchKernelGGL(k_reduce, dim3(nval), dim3(kBlock), 0, s, nblk, part, out, nval_p, gate);
+  hipLaunchKernelGGL(k_reduce, dim3(nval), dim3(kBlock), 0, s, nblk, part, out, nval_p, per, gate);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -468,12 +468,12 @@ __global__ __launch_bounds__(kBlock) void k_ctl(LbdCtl* __restrict__ gc, char* g
                                                 const double* __restrict__ part, int nb) {
   __shared__ LbdCtlLds c;
   __shared__ LbdCtlRef cg;
-  __shared__ double lds[(kBlock / kWave) * 2];
+  __shared__ double lds[(kBlock / kWave) * 3];
   if (gc->phase != want_phase || gc->j != want_j) return;
-  const bool two = (kind == CTL_V_SPMV || kind == CTL_V_ELR || kind == CTL_U_SPMV ||
-                    kind == CTL_U_ELR);
+  const bool three = kind >= CTL_ZV_SPMV;
+  const bool two = three || (kind != CTL_V_REO && kind != CTL_U_REO);
   ctl_stage_body(gc, garr, cap, want_j, kind, part, nb, two ? part + nb : nullptr, nb, c, cg,
-                 lds);
+                 lds, three ? part + 2 * nb : nullptr);
 }
 
 int launch_ctl(hipStream_t s, LbdCtl* c, void* arrays, int cap, int kind, int want_phase,

@@ -64,6 +64,7 @@ struct alignas(16) LbdCtl {
   double alpha, beta, anorm, amax, numax, mumax, rnorm;
   int elr_i;
   double elr_s;       // coefficient of the pending ELR update
+  double elr_im;      // its imaginary part (complex bases)
   int reo_try, reo_k, reo_ncols, reo_nd;
   double reo_norm0;   // ||w|| before the current CGS pass
   int vscale, uscale; // pending 1/alpha, 1/beta scalings of v_j, u_{j+1}
@@ -520,6 +521,52 @@ __host__ __device__ inline void ctl_u_reo_s(C& c, double s2) {
   }
 }
 
+// ---- complex bases (complex16/zlanbpro.F) ----
+// sr, si: real and imaginary part of v_{j-1}^H v_j.  The extended local
+// reorthogonalization of the complex tree (:316-335 for v, :449-466 for u)
+// leaves B alone, its coefficient being complex; the stages are the real ones
+// otherwise.
+template <class C>
+__host__ __device__ inline void zctl_v_spmv_s(C& c, double s2, double sr, double si) {
+  c.elr_im = si;
+  ctl_v_spmv_s(c, s2, sr);
+}
+template <class C>
+__host__ __device__ inline void zctl_u_spmv_s(C& c, double s2, double sr, double si) {
+  c.elr_im = si;
+  ctl_u_spmv_s(c, s2, sr);
+}
+template <class C>
+__host__ __device__ inline void zctl_v_elr_s(C& c, double ns2, double sr, double si) {
+#pragma clang fp contract(off)
+  const double sn = sqrt(ns2);
+  c.elr_im = si;
+  c.elr_i++;
+  if (sn >= c.kappa * c.alpha || c.elr_i >= c.elr) {
+    c.nu[c.j - 1] = c.eps;
+    c.alpha = sn;
+    ctl_v_fin(c);
+  } else {
+    c.alpha = sn;
+    c.elr_s = sr;
+  }
+}
+template <class C>
+__host__ __device__ inline void zctl_u_elr_s(C& c, double ns2, double sr, double si) {
+#pragma clang fp contract(off)
+  const double sn = sqrt(ns2);
+  c.elr_im = si;
+  c.elr_i++;
+  if (sn >= c.kappa * c.beta || c.elr_i >= c.elr) {
+    c.mu[c.j] = c.eps;
+    c.beta = sn;
+    ctl_u_fin(c);
+  } else {
+    c.beta = sn;
+    c.elr_s = sr;
+  }
+}
+
 // Runs a pending omega update serially, then the rest of its step.
 template <class C>
 __host__ __device__ inline void ctl_resume(C& c) {
@@ -567,6 +614,26 @@ __host__ __device__ inline void ctl_u_elr(C& c, double ns2, double nsd) {
 template <class C>
 __host__ __device__ inline void ctl_u_reo(C& c, double s2) {
   ctl_u_reo_s(c, s2);
+  ctl_resume(c);
+}
+template <class C>
+__host__ __device__ inline void zctl_v_spmv(C& c, double s2, double sr, double si) {
+  zctl_v_spmv_s(c, s2, sr, si);
+  ctl_resume(c);
+}
+template <class C>
+__host__ __device__ inline void zctl_u_spmv(C& c, double s2, double sr, double si) {
+  zctl_u_spmv_s(c, s2, sr, si);
+  ctl_resume(c);
+}
+template <class C>
+__host__ __device__ inline void zctl_v_elr(C& c, double ns2, double sr, double si) {
+  zctl_v_elr_s(c, ns2, sr, si);
+  ctl_resume(c);
+}
+template <class C>
+__host__ __device__ inline void zctl_u_elr(C& c, double ns2, double sr, double si) {
+  zctl_u_elr_s(c, ns2, sr, si);
   ctl_resume(c);
 }
 

@@ -297,6 +297,30 @@ int lbd_begin(I& im, int k0, int k_in, double* alpha_, double* beta_, double* rn
   return PK_OK;
 }
 
+// Steps of the call from the state in e->hctl until it is done: device
+// chains from PH_V_SPMV (device), host execution of every other phase.
+template <class I>
+int lbd_loop(I& im, bool device) {
+  Engine* e = im.e;
+  LbdCtlRef& c = *e->hctl;
+  while (c.phase != PH_DONE) {
+    if (device && c.phase == PH_V_SPMV) {
+      const int j_before = c.j;
+      PK_TRY(im.run_device(c));
+      // A chain always advances at least one phase; if it did not, finish
+      // the step on the host rather than enqueue the same chain again.
+      if (c.phase != PH_V_SPMV || c.j != j_before) continue;
+    }
+    // a chain that stopped in a CGS phase ran out of passes: hold two
+    // passes in the engine's later chains
+    if (device && e->tries_auto && e->dev_tries < 2 &&
+        (c.phase == PH_V_REO || c.phase == PH_U_REO))
+      e->dev_tries = 2;
+    PK_TRY(lbd_host_phase(im, c));
+  }
+  return PK_OK;
+}
+
 // End of the call: outputs in the reference's places (dlanbpro.F:540-548).
 template <class I>
 int lbd_end(I& im, int k0, int* kp, double* alpha_, double* beta_, double* rnorm,
