@@ -314,6 +314,9 @@ int pk_batch_bsvd(pk_batch_t batch, int nb, const int* n, const double* d, const
                   int ld, double* sigma, double* bottom);
 int pk_bsvd_batch(int nb, const int* n, const double* d, const double* e, int ld, double* sigma,
                   double* bottom);
+/* ||U(:,1)|| of the first nb problems to nrm (host), all in flight together
+ * (pk_lbd_nrm2 of each one's own engine, bit for bit). */
+int pk_batch_nrm2(pk_batch_t batch, int nb, double* nrm);
 /* pk_lbd_lanbpro for every problem i with active[i] != 0: k0[i] -> k[i]
  * steps; alpha[i], beta[i] its B(:,1), B(:,2); rnorm[i]; doption(4*i+1:
  * 4*i+3) its delta, eta, anorm; ioption shared; ierr[i]. */

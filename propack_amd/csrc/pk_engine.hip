@@ -217,18 +217,27 @@ struct Impl {
     return PK_OK;
   }
 
+  // y = op(A) x - c * yprev by the device operator, enqueued; the number of
+  // slots of its two sums in part.
+  int apply_op(char trans, const T* x, T* y, const T* yprev, double c) {
+    const bool tr = (trans == 't' || trans == 'T');
+    hipEvent_t t0 = tstart(tr ? KC_SPMV_T : KC_SPMV_N);
+    const int nb = csr_apply<T>(e->op, strm, trans, x, y, yprev, sval(c), e->part, Gate{},
+                                e->sw_y, e->sw_l, e->sw_y_len);
+    PK_LAUNCH(nb);
+    tstop(t0, tr ? KC_SPMV_T : KC_SPMV_N, spmv_bytes(tr, yprev != nullptr),
+          2.0 * static_cast<double>(e->op->nnz));
+    return nb;
+  }
+
   // y = op(A) x - c * yprev; *s2 = ||y||^2, *sd = yprev.y (0 without yprev).
   int apply(char trans, const T* x, T* y, const T* yprev, double c, double* s2, double* sd) {
     const bool tr = (trans == 't' || trans == 'T');
     const long long rows_out = tr ? e->n : e->m, rows_in = tr ? e->m : e->n;
     int nb;
     if (e->op) {
-      hipEvent_t t0 = tstart(tr ? KC_SPMV_T : KC_SPMV_N);
-      nb = csr_apply<T>(e->op, strm, trans, x, y, yprev, sval(c), e->part, Gate{}, e->sw_y,
-                        e->sw_l, e->sw_y_len);
-      PK_LAUNCH(nb);
-      tstop(t0, tr ? KC_SPMV_T : KC_SPMV_N, spmv_bytes(tr, yprev != nullptr),
-            2.0 * static_cast<double>(e->op->nnz));
+      nb = apply_op(trans, x, y, yprev, c);
+      PK_TRY(nb);
     } else if (e->aprod) {
       PK_TRY(host_apply(trans, x, y, rows_in, rows_out));
       if (yprev)
@@ -366,6 +375,22 @@ struct Impl {
 
   // dgetu0 (double/dgetu0.F:11-89) writing op(A) x into u0 (device), then
   // orthogonalizing against basis(:, 1:j).  Returns ierr (0 or -1).
+  // The work of getu0's try itry on the device operator, enqueued: x random,
+  // u0 = op(A) x, the squares of their norms to hred[2] and hred[0].
+  int u0_start(bool tn, int itry, T* u0) {
+    const long long rsize = tn ? e->n : e->m;
+    T* x = scratch(0);
+    PK_LAUNCH(launch_larnv_pm1<T>(strm, rsize, x, (itry - 1) * rsize));
+    const int na = launch_norm<T>(strm, rsize, x, e->part);
+    PK_LAUNCH(na);
+    PK_LAUNCH(launch_reduce(strm, 1, na, e->part, e->red + 2, Gate{}));
+    const int nb = apply_op(tn ? 'n' : 't', x, u0, nullptr, 0.0);
+    PK_TRY(nb);
+    PK_LAUNCH(launch_reduce(strm, 2, nb, e->part, e->red, Gate{}));
+    PK_HIP(hipMemcpyAsync(e->hred, e->red, sizeof(double) * 3, hipMemcpyDeviceToHost, strm));
+    return PK_OK;
+  }
+
   int getu0(char transa, int j, int ntry, T* u0, double* u0norm, T* basis, long long ld,
             double* anormest, int* ierr) {
     const bool tn = (transa == 'n' || transa == 'N');
@@ -377,11 +402,20 @@ struct Impl {
     for (int itry = 1; itry <= ntry; ++itry) {
       // DLARNV advances the seed DGETU0 set once per call (double/dgetu0.F:
       // 47-50,67): try t continues the sequence at element (t-1)*rsize
-      PK_LAUNCH(launch_larnv_pm1<T>(strm, rsize, x, (itry - 1) * rsize));
-      double nrm;
-      PK_TRY(nrm2(x, rsize, &nrm));
-      double s2, sd;
-      PK_TRY(apply(tn ? 'n' : 't', x, u0, nullptr, 0.0, &s2, &sd));
+      double nrm, s2, sd;
+      if (e->op && rsize > 0) {  // one wait for both norms
+        if (!e->u0_started) PK_TRY(u0_start(tn, itry, u0));
+        e->u0_started = false;
+        PK_HIP(stream_wait(strm));
+        e->cnt.nsync++;
+        PK_TRY(resolve_timers());
+        s2 = e->hred[0];
+        nrm = std::sqrt(e->hred[2]);
+      } else {
+        PK_LAUNCH(launch_larnv_pm1<T>(strm, rsize, x, (itry - 1) * rsize));
+        PK_TRY(nrm2(x, rsize, &nrm));
+        PK_TRY(apply(tn ? 'n' : 't', x, u0, nullptr, 0.0, &s2, &sd));
+      }
       e->cnt.nopx++;
       *u0norm = std::sqrt(s2);
       *anormest = *u0norm / nrm;
@@ -1055,6 +1089,21 @@ struct ZImpl {
 };
 
 // Pieces of a DLANBPRO call for the batched step engine (pk_batch.hip).
+// engine_lanbpro_prepare enqueues the norm estimate that a call from k0 = 0
+// with a start vector begins with (lbd_begin's getu0), so that the calls of
+// many engines have theirs in flight together; engine_lanbpro_begin takes it.
+int engine_lanbpro_prepare(Engine* e, int k0, double rnorm) {
+  e->u0_started = false;
+  if (prec_is_complex(e->prec) || !e->op || k0 != 0 || rnorm == 0.0 || e->m < 1 || e->n < 1)
+    return PK_OK;
+  const bool tn = e->n > e->m;
+  const int rc = e->prec == PK_F64
+                     ? Impl<double>(e).u0_start(tn, 1, Impl<double>(e).scratch(1))
+                     : Impl<float>(e).u0_start(tn, 1, Impl<float>(e).scratch(1));
+  e->u0_started = rc == PK_OK;
+  return rc;
+}
+
 int engine_lanbpro_begin(Engine* e, int k0, int k, double* alpha, double* beta, double* rnorm,
                          double* doption, const int* ioption, int* ierr, bool* finished) {
   if (k > e->kmax || k0 < 0 || k0 > k) {
@@ -1065,11 +1114,31 @@ int engine_lanbpro_begin(Engine* e, int k0, int k, double* alpha, double* beta, 
     set_error("batched steps take real engines only");
     return PK_ERR_NOTSUP;
   }
-  if (e->prec == PK_F64)
-    return Impl<double>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption, ierr,
-                                         finished);
-  return Impl<float>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption, ierr,
-                                      finished);
+  const int rc = e->prec == PK_F64
+                     ? Impl<double>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption,
+                                                     ierr, finished)
+                     : Impl<float>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption,
+                                                    ierr, finished);
+  e->u0_started = false;
+  return rc;
+}
+
+// ||U(:,1)|| of a real engine in two halves: the kernels and the copy
+// enqueued on its stream, then the wait.
+int engine_nrm2_start(Engine* e) {
+  const int nb = e->prec == PK_F64
+                     ? launch_norm<double>(e->stream, e->m, static_cast<double*>(e->u()), e->part)
+                     : launch_norm<float>(e->stream, e->m, static_cast<float*>(e->u()), e->part);
+  PK_LAUNCH(nb);
+  PK_LAUNCH(launch_reduce(e->stream, 1, nb, e->part, e->red, Gate{}));
+  PK_HIP(hipMemcpyAsync(e->hred, e->red, sizeof(double), hipMemcpyDeviceToHost, e->stream));
+  return PK_OK;
+}
+int engine_nrm2_finish(Engine* e, double* out) {
+  PK_HIP(hipStreamSynchronize(e->stream));
+  e->cnt.nsync++;
+  *out = std::sqrt(e->hred[0]);
+  return PK_OK;
 }
 
 int engine_lanbpro_loop(Engine* e) {

@@ -313,6 +313,7 @@ struct Engine {
   double* hB = nullptr;              // pinned host staging
   hipEvent_t evB = nullptr;          // the last copy out of hB (reuse guard)
   void* vec = nullptr;               // scratch vector, max(m, n)
+  bool u0_started = false;           // a norm estimate is in flight (engine_lanbpro_prepare)
   double* sw_y = nullptr;            // SpMV running row sums (csr_ywork(op) at creation)
   long long sw_y_len = 0;
   double* sw_l = nullptr;            // SpMV long-row partial sums (csr_lwork(op))
@@ -345,6 +346,9 @@ struct Engine {
 // outputs), so that several engines can run their steps together.
 int engine_lanbpro_begin(Engine* e, int k0, int k, double* alpha, double* beta, double* rnorm,
                          double* doption, const int* ioption, int* ierr, bool* finished);
+int engine_lanbpro_prepare(Engine* e, int k0, double rnorm);
+int engine_nrm2_start(Engine* e);
+int engine_nrm2_finish(Engine* e, double* out);
 int engine_lanbpro_loop(Engine* e);
 int engine_lanbpro_end(Engine* e, int k0, int* kp, double* alpha, double* beta, double* rnorm,
                        double* doption, int* ierr);

@@ -18,7 +18,7 @@ module pk_drivers
   implicit none
   private
   public :: lansvd_core, lansvd_irl_core, add_timing, irl_begin, irl_after, irl_end, &
-            irl_pre_svd, irl_host_svd, irl_post_svd
+            irl_pre_svd, irl_host_svd, irl_post_svd, irl_ritz_svd, irl_ritz_update
 
   ! External LAPACK (host): bidiagonal SVD.
   interface
@@ -47,6 +47,11 @@ module pk_drivers
     ! defer: the restart GEMMs are left to the caller (the batched driver
     ! runs every problem's in one launch); pending: this pass left them
     logical :: defer = .false., pending = .false.
+    ! ritz: the Ritz factors are in pm (rows mstart.. of P^T M^T) and qm
+    ! (rows of Q^T), ritz_done: the Ritz vectors are formed (the batched
+    ! driver: irl_ritz_svd per problem, one grouped product for all)
+    logical :: ritz = .false., ritz_done = .false.
+    integer :: mstart = 1
     integer(c_long_long) :: st0(8) = 0
     double precision, allocatable :: alpha(:), beta(:), a1(:), b1(:), wb(:), shift(:), &
                                      pm(:, :), qm(:, :), wrk(:), sig(:), bd(:)
@@ -102,23 +107,21 @@ contains
     if (nsing_set >= 0) nsing = nsing_set
   end subroutine
 
-  ! Ritz vectors from A V_dim = U_{dim+1} B_dim (DRITZVEC): B = M [R; 0]
-  ! by Givens QR, R = P S Q^T by divide and conquer (DBDSDC), then
-  ! U <- U (P^T M^T)^T rows, V <- V Q on the device.
-  subroutine ritzvec(which, jobu, jobv, m, n, k, dim, d, e, eng, info)
-    character(len=1), intent(in) :: which, jobu, jobv
+  ! The small factors of the Ritz vectors from A V_dim = U_{dim+1} B_dim
+  ! (DRITZVEC): B = M [R; 0] by Givens QR, R = P S Q^T by divide and conquer
+  ! (DBDSDC); x(1:dim, 1:dim+1) = P^T M^T, qt = Q^T, whose rows from mstart
+  ! on belong to the k wanted triplets.
+  subroutine ritz_factors(which, jobu, m, n, k, dim, d, e, x, qt, mstart)
+    character(len=1), intent(in) :: which, jobu
     integer, intent(in) :: m, n, k, dim
     double precision, intent(inout) :: d(*), e(*)
-    type(c_ptr), intent(in) :: eng
-    integer, intent(out) :: info
-    double precision, allocatable :: mt(:, :), qt(:, :), p(:, :), x(:, :), wrk(:)
+    double precision, intent(out) :: x(dim + 1, dim + 1), qt(dim, dim)
+    integer, intent(out) :: mstart
+    double precision, allocatable :: mt(:, :), p(:, :), wrk(:)
     integer, allocatable :: iwk(:)
     double precision :: c1, c2, dd(1)
-    integer :: id(1), mstart, lapinfo
-    integer(c_int) :: rc
-    info = 0
-    if (k < 1) return
-    allocate(mt(dim + 1, dim + 1), qt(dim, dim), p(dim, dim), x(dim + 1, dim + 1))
+    integer :: id(1), lapinfo
+    allocate(mt(dim + 1, dim + 1), p(dim, dim))
     allocate(wrk(3 * dim * dim + 4 * dim + 8), iwk(8 * dim + 8))
     mt = 0d0; qt = 0d0; p = 0d0; x = 0d0
     c1 = 0d0; c2 = 0d0
@@ -131,6 +134,23 @@ contains
     else
       mstart = 1
     end if
+  end subroutine
+
+  ! Ritz vectors: the factors, then U <- U (P^T M^T)^T rows, V <- V Q on the
+  ! device.
+  subroutine ritzvec(which, jobu, jobv, m, n, k, dim, d, e, eng, info)
+    character(len=1), intent(in) :: which, jobu, jobv
+    integer, intent(in) :: m, n, k, dim
+    double precision, intent(inout) :: d(*), e(*)
+    type(c_ptr), intent(in) :: eng
+    integer, intent(out) :: info
+    double precision, allocatable :: qt(:, :), x(:, :)
+    integer :: mstart
+    integer(c_int) :: rc
+    info = 0
+    if (k < 1) return
+    allocate(qt(dim, dim), x(dim + 1, dim + 1))
+    call ritz_factors(which, jobu, m, n, k, dim, d, e, x, qt, mstart)
     if (lower1(jobu) == 'y') then
       ! U(:,1:k) <- U(:,1:dim+1) * X(mstart:mstart+k-1, :)^T
       rc = pk_lbd_update(eng, 'u', 't', dim + 1, k, x(mstart, 1), dim + 1)
@@ -301,7 +321,7 @@ contains
 
   ! Driver setup up to the first DLANBPRO call (double/dlansvd_irl.F:160-206).
   subroutine irl_begin(st, which, jobu, jobv, m, n, dim, p, neig, maxiter, eng, eps, tolin, &
-                       doption, ioption)
+                       doption, ioption, norm0)
     type(irl_state), intent(inout) :: st
     character(len=1), intent(in) :: which, jobu, jobv
     integer, intent(in) :: m, n, dim, p, neig, maxiter
@@ -309,6 +329,7 @@ contains
     double precision, intent(in) :: eps, tolin
     double precision, intent(in) :: doption(*)
     integer, intent(in) :: ioption(*)
+    double precision, intent(in), optional :: norm0  ! ||U(:,1)||, where the caller has it
     integer(c_int) :: rc, ierr_c
 
     st%eng = eng
@@ -348,7 +369,12 @@ contains
     st%done = .false.
     st%failed = .false.
 
-    rc = pk_lbd_nrm2(eng, 'u', 1, st%rnorm)
+    rc = PK_OK
+    if (present(norm0)) then
+      st%rnorm = norm0
+    else
+      rc = pk_lbd_nrm2(eng, 'u', 1, st%rnorm)
+    end if
     if (rc == PK_OK .and. st%rnorm == 0d0) &
       rc = pk_lbd_getu0(eng, 'n', 0, 1, st%rnorm, ioption(1), st%anorm, ierr_c)
     if (rc /= PK_OK) then
@@ -527,6 +553,47 @@ contains
     st%done = .not. (st%nconv < st%neig .and. st%iter < st%maxiter)
   end subroutine
 
+  ! Whether the solve ends with Ritz vectors (double/dlansvd_irl.F:396).
+  logical function irl_vectors(st)
+    type(irl_state), intent(in) :: st
+    irl_vectors = .not. st%failed .and. (st%nconv >= st%neig .or. st%info > 0) .and. &
+                  (lower1(st%jobu) == 'y' .or. lower1(st%jobv) == 'y')
+  end function
+
+  ! The Ritz factors of a finished problem (ritzvec's host part), into pm, qm.
+  subroutine irl_ritz_svd(st)
+    type(irl_state), intent(inout) :: st
+    st%ritz = .false.
+    if (.not. irl_vectors(st) .or. st%nconv < 1) return
+    if (size(st%pm, 1) /= st%dim + 1) then  ! dim lowered at an invariant subspace
+      deallocate(st%pm, st%qm)
+      allocate(st%pm(st%dim + 1, st%dim + 1), st%qm(st%dim, st%dim))
+    end if
+    st%a1 = st%alpha
+    st%b1 = st%beta
+    call ritz_factors(st%which, st%jobu, st%m, st%n, st%nconv, st%dim, st%a1, st%b1, st%pm, &
+                      st%qm, st%mstart)
+    st%ritz = .true.
+  end subroutine
+
+  ! One problem's Ritz product on its own engine: side 'u' or 'v'.
+  subroutine irl_ritz_update(st, side)
+    type(irl_state), intent(inout) :: st
+    character(len=1), intent(in) :: side
+    integer(c_int) :: rc
+    if (side == 'u') then
+      rc = pk_lbd_update(st%eng, 'u', 't', st%dim + 1, st%nconv, st%pm(st%mstart, 1), &
+                         size(st%pm, 1))
+    else
+      rc = pk_lbd_update(st%eng, 'v', 't', st%dim, st%nconv, st%qm(st%mstart, 1), &
+                         size(st%qm, 1))
+    end if
+    if (rc == PK_OK) rc = pk_lbd_sync(st%eng)
+    if (rc == PK_OK) return
+    st%info = rc
+    st%ritz_done = .true.  ! as far as it got
+  end subroutine
+
   ! Ritz vectors and outputs (double/dlansvd_irl.F:396-418).
   subroutine irl_end(st, sigma, bnd, dim, neig, info, doption)
     type(irl_state), intent(inout) :: st
@@ -534,13 +601,11 @@ contains
     integer, intent(inout) :: dim, neig
     integer, intent(out) :: info
     integer :: jj
-    logical :: vectors
 
     doption(1:4) = st%dopt
     info = st%info
     if (st%failed) return  ! an engine error: outputs as they were
-    vectors = lower1(st%jobu) == 'y' .or. lower1(st%jobv) == 'y'
-    if ((st%nconv >= st%neig .or. st%info > 0) .and. vectors) then
+    if (irl_vectors(st) .and. .not. st%ritz_done) then
       st%a1 = st%alpha
       st%b1 = st%beta
       call ritzvec(st%which, st%jobu, st%jobv, st%m, st%n, st%nconv, st%dim, st%a1, st%b1, &
@@ -582,9 +647,27 @@ module pk_batch_par
       type(c_funptr), value :: fn
       type(c_ptr), value :: ctx
     end subroutine
+    ! threads of the calling thread's MKL calls (0: the process's number);
+    ! returns the number before
+    integer(c_int) function mkl_set_num_threads_local(nt) &
+        bind(C, name='MKL_Set_Num_Threads_Local')
+      import :: c_int
+      integer(c_int), value :: nt
+    end function
   end interface
 
 contains
+
+  ! The small SVDs of a finished problem's Ritz vectors.  MKL runs each on the
+  ! one thread it is called from: the problems are the parallelism here.
+  subroutine ritz_one(st)
+    type(irl_state), intent(inout) :: st
+    integer(c_int) :: was
+    if (.not. st%done) return
+    was = mkl_set_num_threads_local(1_c_int)
+    call irl_ritz_svd(st)
+    was = mkl_set_num_threads_local(was)
+  end subroutine
 
   subroutine after_one(ctx, i0) bind(C)
     type(c_ptr), value :: ctx
@@ -597,6 +680,7 @@ contains
     c%st(i)%rnorm = c%rn(i)
     c%st(i)%dopt = c%dop(:, i)
     call irl_after(c%st(i), c%kk(i), c%ierr(i))
+    call ritz_one(c%st(i))
   end subroutine
 
   ! The same in two halves around the device bidiagonal SVDs.
@@ -623,6 +707,7 @@ contains
     if (c%active(i) == 0) return
     if (c%dev(i) == 0) call irl_host_svd(c%st(i))
     call irl_post_svd(c%st(i))
+    call ritz_one(c%st(i))
   end subroutine
 
 end module pk_batch_par
@@ -744,6 +829,12 @@ integer(c_int) function pk_lansvd_irl_batch(nb, engs, batch, which, jobu, jobv, 
       integer(c_int) :: sel(*), kdim(*), ncols(*), ldb(*)
       type(c_ptr) :: bm(*)
     end function
+    integer(c_int) function pk_batch_nrm2(b, nb, nrm) bind(C, name='pk_batch_nrm2')
+      import :: c_int, c_ptr, c_double
+      type(c_ptr), value :: b
+      integer(c_int), value :: nb
+      real(c_double) :: nrm(*)
+    end function
   end interface
   integer, parameter :: bsvd_max = 128  ! largest order of the device bidiagonal SVD
   type(irl_state), allocatable, target :: st(:)
@@ -756,6 +847,7 @@ integer(c_int) function pk_lansvd_irl_batch(nb, engs, batch, which, jobu, jobv, 
   type(after_ctx), target :: ctx
   integer :: i, j, m, n, rc, dd, ne, nd, ldb
   integer(c_int) :: usedev
+  logical :: normed
   double precision :: eps, dummy(4), c1
 
   pk_lansvd_irl_batch = PK_OK
@@ -770,14 +862,21 @@ integer(c_int) function pk_lansvd_irl_batch(nb, engs, batch, which, jobu, jobv, 
   end if
   ldb = max(dim, 1)
   if (usedev /= 0) allocate(bd(ldb, nb), be(ldb, nb), bs(ldb, nb), bb(ldb, nb))
+  ! the start vectors' norms, every engine's in flight together
+  normed = pk_batch_nrm2(batch, nb, rn) == PK_OK
   do i = 1, nb
     call engine_shape(engs(i), m, n, eps, rc)
     if (rc /= 0) then
       pk_lansvd_irl_batch = rc
       return
     end if
-    call irl_begin(st(i), which, jobu, jobv, m, n, dim, p, neig, maxiter, engs(i), eps, tolin, &
-                   doption, ioption)
+    if (normed) then
+      call irl_begin(st(i), which, jobu, jobv, m, n, dim, p, neig, maxiter, engs(i), eps, tolin, &
+                     doption, ioption, rn(i))
+    else
+      call irl_begin(st(i), which, jobu, jobv, m, n, dim, p, neig, maxiter, engs(i), eps, tolin, &
+                     doption, ioption)
+    end if
     st(i)%defer = .true.
   end do
   do while (any(.not. st(:)%done))
@@ -854,6 +953,11 @@ integer(c_int) function pk_lansvd_irl_batch(nb, engs, batch, which, jobu, jobv, 
     call pkx_parallel_for(nb, c_funloc(post_one), c_loc(ctx))
     call restart_gemms()
   end do
+  ! Ritz vectors, one grouped product per side (after_one and post_one left
+  ! each finished problem's factors)
+  if (lower1(jobu) == 'y') call ritz_gemms('u')
+  if (lower1(jobv) == 'y') call ritz_gemms('v')
+  st(:)%ritz_done = st(:)%ritz_done .or. st(:)%ritz
   do i = 1, nb
     dd = dim
     ne = neig
@@ -862,6 +966,35 @@ integer(c_int) function pk_lansvd_irl_batch(nb, engs, batch, which, jobu, jobv, 
     nconv(i) = ne
   end do
 contains
+  ! U(:,1:k) <- U(:,1:dim+1) X^T or V(:,1:k) <- V(:,1:dim) Q of every problem
+  ! with Ritz factors; where the grouped product is not to be had (a spare
+  ! basis that does not fit, say), each problem's own, with its own outcome.
+  subroutine ritz_gemms(side)
+    character(len=1), intent(in) :: side
+    integer :: nu, q
+    nu = 0
+    do q = 1, nb
+      if (.not. st(q)%ritz .or. st(q)%ritz_done) cycle
+      nu = nu + 1
+      usel(nu) = q - 1
+      unc(nu) = st(q)%nconv
+      if (side == 'u') then
+        ukd(nu) = st(q)%dim + 1
+        uld(nu) = size(st(q)%pm, 1)
+        upm(nu) = c_loc(st(q)%pm(st(q)%mstart, 1))
+      else
+        ukd(nu) = st(q)%dim
+        uld(nu) = size(st(q)%qm, 1)
+        upm(nu) = c_loc(st(q)%qm(st(q)%mstart, 1))
+      end if
+    end do
+    if (nu == 0) return
+    if (pk_batch_update(batch, nu, usel, side, 't', ukd, unc, upm, uld) == PK_OK) return
+    do q = 1, nu
+      call irl_ritz_update(st(usel(q) + 1), side)
+    end do
+  end subroutine
+
   ! The restart GEMMs this pass left (double/dlansvd_irl.F:387-395) for every
   ! problem at once: U(:,1:k+1) <- U(:,1:dim+1) P and V(:,1:k) <- V(:,1:dim) Q,
   ! one grouped launch each.
