@@ -24,6 +24,15 @@ constexpr int kBlock = 256;        // threads per workgroup for streaming kernel
 constexpr int kMaxBlocks = 2048;   // fixed upper bound on the streaming grid (8 per CU)
 constexpr int kMaxCols = 512;      // most basis columns one reorthogonalization can touch
 
+// A device pointer that a kernel read from memory, known to the compiler to
+// be global: it takes such pointers for generic ones, whose loads and stores
+// also hold up the LDS counter (the batched kernels read all of theirs from
+// tables).
+template <typename X>
+__device__ __forceinline__ X* as_global(X* p) {
+  return (X*)(__attribute__((address_space(1))) X*)reinterpret_cast<uintptr_t>(p);
+}
+
 // Scalar operand of a kernel: read from device memory when p != nullptr
 // (device-resident control), otherwise the by-value v (host control).
 struct Scal {

@@ -190,8 +190,10 @@ __global__ __launch_bounds__(kSortThreads) void k_spmv_sorted_cp(
   extern __shared__ double prod_dyn[];
   __shared__ double lds[(kSortThreads / kWave) * 2];
   const int p = mp.x;
-  spmv_sorted_body<VT, T, G>(table->desc[p][mp.y], table->rp[p], table->sci[p],
-                             static_cast<const VT*>(table->sva[p]), table->spos[p],
+  spmv_sorted_body<VT, T, G>(as_global(table->desc[p])[mp.y], as_global(table->rp[p]),
+                             as_global(table->sci[p]),
+                             as_global(static_cast<const VT*>(table->sva[p])),
+                             as_global(table->spos[p]),
                              table->col0[p], table->pbits[p], x, nullptr, nullptr, 0.0,
                              nullptr, nullptr, nullptr, nullptr,
                              ypart + static_cast<long long>(p) * rows, 0, prod_dyn, lds);
@@ -672,9 +674,9 @@ __global__ __launch_bounds__(kWave * kGemmWaves, 2) void k_gemm_lds_group(
   const GemmItem it = items[blockIdx.x];
   const long long L = it.L, lda = it.lda, ldc = it.ldc;
   const int kdim = it.kdim, kpad = it.kpad, ldb = it.ldb, ncols = it.ncols;
-  const T* __restrict__ A = static_cast<const T*>(it.A);
-  const double* __restrict__ B = it.B;
-  T* __restrict__ C = static_cast<T*>(it.C);
+  const T* __restrict__ A = as_global(static_cast<const T*>(it.A));
+  const double* __restrict__ B = as_global(it.B);
+  T* __restrict__ C = as_global(static_cast<T*>(it.C));
   extern __shared__ double Bs[];  // Bs[j * kpad + k] = B(k, j), zero outside kdim x ncols
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
   const int li = lane % 16, lk = lane / 16;
