@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void k_bspmv_vec(const BProb* __restrict__ 
 // kSortThreads workgroup per descriptor, the launch's largest block cap of
 // dynamic LDS.
 template <typename VT, typename T>
-__global__ __launch_bounds__(kSortThreads) void k_bspmv_sorted(
+__global__ __launch_bounds__(kSortThreads, 8) void k_bspmv_sorted(
     const BProb* __restrict__ probs, const BPanel* __restrict__ panels,
     const int4* __restrict__ desc, const BWork* __restrict__ work, int tr, int p, int J,
     int phase, double* __restrict__ part, int Q) {

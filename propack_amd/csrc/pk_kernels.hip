@@ -126,7 +126,7 @@ int launch_spmv_rb(hipStream_t s, int nblk, const int4* desc, int nlong, const i
 // (spmv_sorted_body); the products of a block take cap doubles of dynamic
 // LDS.  Partial slots and the long-row fix-up as in k_spmv_rb.
 template <typename VT, typename T, int G>
-__global__ __launch_bounds__(kSortThreads) void k_spmv_sorted(
+__global__ __launch_bounds__(kSortThreads, 8) void k_spmv_sorted(
     const int4* __restrict__ desc, const int* __restrict__ rp, const int* __restrict__ sci,
     const VT* __restrict__ sva, const unsigned short* __restrict__ spos, int col0, int pbits,
     const T* __restrict__ x, T* __restrict__ y, const T* __restrict__ yprev, Scal coef,
@@ -181,7 +181,7 @@ int launch_spmv_sorted(hipStream_t s, int nblk, const int4* desc, int nlong, con
 
 // -------------------------------------------- sorted SpMV, panels at once --
 template <typename VT, typename T, int G>
-__global__ __launch_bounds__(kSortThreads) void k_spmv_sorted_cp(
+__global__ __launch_bounds__(kSortThreads, 8) void k_spmv_sorted_cp(
     const SortPanels* __restrict__ table, const int2* __restrict__ map, long long rows,
     const T* __restrict__ x, double* __restrict__ ypart, Gate gate) {
   if (gate.off()) return;
