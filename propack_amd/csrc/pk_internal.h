@@ -162,7 +162,7 @@ int csr_apply(const CsrOp* op, hipStream_t s, char trans, const T* x, T* y, cons
               Scal coef, double* part, Gate gate, double* ywork = nullptr,
               double* lwork = nullptr, long long ywork_len = 0);
 // Long-row partial sums one panel can need, for any layout of op: a row of
-// len > kSpmvCap nonzeros has ceil(len / kLongChunk) <= len / kSpmvCap chunks.
+// len > kSpmvCap nonzeros has at most len / kSpmvCap chunks (partition).
 inline long long csr_lwork(const CsrOp* op) { return op->nnz / 1024 + 2; }
 
 // ---- tile layout (pk_tile.hip) ----
