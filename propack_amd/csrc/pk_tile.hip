@@ -58,11 +58,16 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Workgroup w runs unit w.  Streams are loaded two groups of U batches ahead,
-// x is gathered one group ahead, in three register stages of a loop unrolled
-// by three (no stage is copied).  Measured at the size above: U = 1 / 2 / 4 / 6
-// 110 / 107 / 117 / 126 us; streams and gathers of one group only, 131 us; two
-// 512-thread workgroups per CU on half the rows each 121-141 us.
+// Workgroup w runs unit w.  Streams and batch bases are loaded three groups of
+// U batches ahead, x is gathered one group ahead, in four register stages of a
+// loop unrolled by four (no stage is copied).  The gathers bound it: without
+// them the 2M x 1M, FP64, 32M directions take 80 us instead of 123 and 111,
+// 1M x 500k, FP32, 16M 25 and 35 instead of 51 and 43; without the adds
+// instead 115 and 111, 45 and 48.  Streams two groups ahead and each base read
+// beside its gather: 1 to 2% longer in FP64, FP32 51.5 and 43.4 us instead of
+// 47.8 and 42.6; x two groups ahead: the same or longer.  U = 1 / 2 / 4 / 6
+// (streams two ahead, first of these) 110 / 107 / 117 / 126 us; two 512-thread
+// workgroups per CU on half the rows each 121-141 us.
 // last: the unit is its rows' only segment; the epilogue y = T(sum - c yprev)
 // and the partials follow.  Otherwise the sums go to ypart[segment].
 template <typename VT, typename T, int U>
@@ -79,47 +84,59 @@ __global__ __launch_bounds__(kTB) void k_spmv_tile(
   const unsigned* __restrict__ w0 = wd + static_cast<long long>(t.b0) * kTB + threadIdx.x;
   const VT* __restrict__ v0 = va + static_cast<long long>(t.b0) * kTB + threadIdx.x;
   const int* __restrict__ bb = base + t.b0;
-  unsigned wa[U], wb[U], wc[U];
-  VT a[U], b[U], c[U];
-  T xa[U], xb[U], xc[U];
+  struct Stage {
+    unsigned w[U];
+    VT v[U];
+    T x[U];
+    int n[U];
+  };
+  Stage a, b, c, d;
   // groups past the end load the last one again and are not added
-  auto load = [&](int g, unsigned(&w)[U], VT(&v)[U]) {
-    const long long o = static_cast<long long>(min(g, ng - 1)) * U * kTB;
-#pragma unroll
-    for (int u = 0; u < U; ++u) w[u] = __builtin_nontemporal_load(w0 + o + u * kTB);
-#pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(v0 + o + u * kTB);
-  };
-  auto gather = [&](int g, const unsigned(&w)[U], T(&xv)[U]) {
+  auto load = [&](int g, Stage& q) {
     const int gb = min(g, ng - 1) * U;
+    const long long o = static_cast<long long>(gb) * kTB;
 #pragma unroll
-    for (int u = 0; u < U; ++u) xv[u] = x[bb[gb + u] + static_cast<int>(w[u] >> kTileRowBits)];
+    for (int u = 0; u < U; ++u) q.w[u] = __builtin_nontemporal_load(w0 + o + u * kTB);
+#pragma unroll
+    for (int u = 0; u < U; ++u) q.v[u] = __builtin_nontemporal_load(v0 + o + u * kTB);
+#pragma unroll
+    for (int u = 0; u < U; ++u) q.n[u] = bb[gb + u];
   };
-  auto add = [&](const unsigned(&w)[U], const VT(&v)[U], const T(&xv)[U]) {
+  auto gather = [&](Stage& q) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) q.x[u] = x[q.n[u] + static_cast<int>(q.w[u] >> kTileRowBits)];
+  };
+  auto add = [&](const Stage& q) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const unsigned r = w[u] & kTilePad;
-      if (r != kTilePad) lds_add(acc + r, static_cast<double>(v[u]) * static_cast<double>(xv[u]));
+      const unsigned r = q.w[u] & kTilePad;
+      if (r != kTilePad)
+        lds_add(acc + r, static_cast<double>(q.v[u]) * static_cast<double>(q.x[u]));
       lds_barrier();
     }
   };
-  load(0, wa, a);
-  load(1, wb, b);
+  load(0, a);
+  load(1, b);
+  load(2, c);
   for (int i = threadIdx.x; i < t.nrows; i += kTB) acc[i] = 0.0;
-  gather(0, wa, xa);
+  gather(a);
   lds_barrier();
   for (int g = 0;;) {
-    gather(g + 1, wb, xb);
-    load(g + 2, wc, c);
-    add(wa, a, xa);
+    gather(b);
+    load(g + 3, d);
+    add(a);
     if (++g >= ng) break;
-    gather(g + 1, wc, xc);
-    load(g + 2, wa, a);
-    add(wb, b, xb);
+    gather(c);
+    load(g + 3, a);
+    add(b);
     if (++g >= ng) break;
-    gather(g + 1, wa, xa);
-    load(g + 2, wb, b);
-    add(wc, c, xc);
+    gather(d);
+    load(g + 3, b);
+    add(c);
+    if (++g >= ng) break;
+    gather(a);
+    load(g + 3, c);
+    add(d);
     if (++g >= ng) break;
   }
   if (!last) {
