@@ -285,7 +285,8 @@ __global__ __launch_bounds__(kBlock) void k_bctl(const BProb* __restrict__ probs
   __shared__ LbdCtlLds c;
   __shared__ LbdCtlRef cg;
   __shared__ double lds[(kBlock / kWave) * 3];
-  if (P.ctl->phase != phase || P.ctl->j != J) return;
+  const int ph = P.ctl->phase, jj = P.ctl->j;
+  if ((ph != phase) | (jj != J)) return;
   const double* pa;
   const double* pb = nullptr;
   int na;
@@ -323,9 +324,9 @@ __global__ __launch_bounds__(kBlock) void k_bgemvt(const BProb* __restrict__ pro
                                                    int J, int phase, double* __restrict__ part,
                                                    int S) {
   const BProb P = prob_at(probs, slice_pid[blockIdx.x]);
-  if (Gate{P.ctl, phase, J, 0}.off()) return;
+  int ncols;
+  if (gated(Gate{P.ctl, phase, J, 0}, &P.ctl->reo_ncols, 0, ncols)) return;
   __shared__ double lds[2][(kBlock / kWave) * kCT];
-  const int ncols = P.ctl->reo_ncols;
   const int* scol = CtlArrays::cols(P.arr, P.cap);
   const long long b = static_cast<long long>(blockIdx.x) - (vside ? P.cn0 : P.cm0);
   const T* basis = static_cast<const T*>(vside ? P.V : P.U);
@@ -341,9 +342,10 @@ __global__ __launch_bounds__(kBlock) void k_breduce(const BProb* __restrict__ pr
                                                     const double* __restrict__ part, int S,
                                                     double* __restrict__ red, int rs) {
   const BProb P = prob_at(probs, blockIdx.x);
-  if (Gate{P.ctl, phase, J, 0}.off()) return;
+  int ncols;
+  if (gated(Gate{P.ctl, phase, J, 0}, &P.ctl->reo_ncols, 0, ncols)) return;
   const int c = blockIdx.y;
-  if (c >= P.ctl->reo_ncols) return;
+  if (c >= ncols) return;
   __shared__ double lds[kBlock / kWave];
   const int s0 = vside ? P.cn0 : P.cm0, ns = vside ? P.ncn : P.ncm;
   const double v = reduce_partials(part + static_cast<long long>(c) * S + s0, ns, lds);
@@ -358,9 +360,9 @@ __global__ __launch_bounds__(kBlock) void k_bgemv(const BProb* __restrict__ prob
                                                   double* __restrict__ part) {
   const int pid = slice_pid[blockIdx.x];
   const BProb P = prob_at(probs, pid);
-  if (Gate{P.ctl, phase, J, 0}.off()) return;
+  int ncols;
+  if (gated(Gate{P.ctl, phase, J, 0}, &P.ctl->reo_ncols, 0, ncols)) return;
   __shared__ double lds[kBlock / kWave];
-  const int ncols = P.ctl->reo_ncols;
   const int* scol = CtlArrays::cols(P.arr, P.cap);
   const double* sh = red + static_cast<long long>(pid) * rs;
   const long long b = static_cast<long long>(blockIdx.x) - (vside ? P.cn0 : P.cm0);

@@ -33,6 +33,13 @@ __device__ __forceinline__ X* as_global(X* p) {
   return (X*)(__attribute__((address_space(1))) X*)reinterpret_cast<uintptr_t>(p);
 }
 
+// Values loaded by the time this is reached: a kernel's scalar loads issued
+// before a branch arrive in one round trip instead of one after the branch.
+template <typename X>
+__device__ __forceinline__ void ready(X x) {
+  asm volatile("" : : "s"(x));
+}
+
 // Scalar operand of a kernel: read from device memory when p != nullptr
 // (device-resident control), otherwise the by-value v (host control).
 struct Scal {

@@ -324,8 +324,8 @@ __global__ __launch_bounds__(kBlock) void k_zgemvt(long long L,
                                                    const typename V2T<R>::type* __restrict__ w,
                                                    double* __restrict__ part, Gate gate) {
   using C2 = typename V2T<R>::type;
-  if (gate.off()) return;
-  const int ncols = ncols_p ? *ncols_p : ncols_v;
+  int ncols;
+  if (gated(gate, ncols_p, ncols_v, ncols)) return;
   __shared__ double lds[(kBlock / kWave) * 2 * kZCols];
   const size_t nb = gridDim.x;
   if (L <= 0) {  // empty vectors: zero projections, no loads
@@ -390,8 +390,8 @@ __global__ __launch_bounds__(kBlock) void k_zgemv_update(long long L,
                                                          typename V2T<R>::type* __restrict__ w,
                                                          double* __restrict__ part, Gate gate) {
   using C2 = typename V2T<R>::type;
-  if (gate.off()) return;
-  const int ncols = ncols_p ? *ncols_p : ncols_v;
+  int ncols;
+  if (gated(gate, ncols_p, ncols_v, ncols)) return;
   __shared__ double lds[kBlock / kWave];
   if (L <= 0) {
     if (threadIdx.x == 0) part[blockIdx.x] = 0.0;

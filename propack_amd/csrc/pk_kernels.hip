@@ -40,10 +40,13 @@ __global__ __launch_bounds__(kBlock) void k_spmv_rb(const int4* __restrict__ des
                                                     const double* __restrict__ yacc_in,
                                                     double* __restrict__ yacc_out, int last,
                                                     Gate gate) {
-  if (gate.off()) return;
+  const int4 d = desc[blockIdx.x];
+  const bool off = gate.off();
+  ready(d.x);
+  if (off) return;
   __shared__ double prod[kSpmvCap];
   __shared__ double lds[(kBlock / kWave) * 2];
-  spmv_rb_body<VT, T, G>(desc[blockIdx.x], rp, ci, va, x, y, yprev, coef.get(),
+  spmv_rb_body<VT, T, G>(d, rp, ci, va, x, y, yprev, coef.get(),
                          part + blockIdx.x, part + nbt + blockIdx.x, lsum, yacc_in, yacc_out,
                          last, prod, lds);
 }
@@ -61,9 +64,12 @@ __global__ __launch_bounds__(kBlock) void k_spmv_vec(const int4* __restrict__ de
                                                      const double* __restrict__ yacc_in,
                                                      double* __restrict__ yacc_out, int last,
                                                      Gate gate) {
-  if (gate.off()) return;
+  const int4 d = desc[blockIdx.x];
+  const bool off = gate.off();
+  ready(d.x);
+  if (off) return;
   __shared__ double lds[(kBlock / kWave) * 2];
-  spmv_vec_body<VT, T, G>(desc[blockIdx.x], rp, ci, va, x, y, yprev, coef.get(),
+  spmv_vec_body<VT, T, G>(d, rp, ci, va, x, y, yprev, coef.get(),
                           part + blockIdx.x, part + nbt + blockIdx.x, lsum, yacc_in, yacc_out,
                           last, lds);
 }
@@ -132,10 +138,13 @@ __global__ __launch_bounds__(kSortThreads, 8) void k_spmv_sorted(
     const T* __restrict__ x, T* __restrict__ y, const T* __restrict__ yprev, Scal coef,
     double* __restrict__ part, int nbt, double* __restrict__ lsum,
     const double* __restrict__ yacc_in, double* __restrict__ yacc_out, int last, Gate gate) {
-  if (gate.off()) return;
+  const int4 d = desc[blockIdx.x];
+  const bool off = gate.off();
+  ready(d.x);
+  if (off) return;
   extern __shared__ double prod_dyn[];
   __shared__ double lds[(kSortThreads / kWave) * 2];
-  spmv_sorted_body<VT, T, G>(desc[blockIdx.x], rp, sci, sva, spos, col0, pbits, x, y, yprev,
+  spmv_sorted_body<VT, T, G>(d, rp, sci, sva, spos, col0, pbits, x, y, yprev,
                              coef.get(),
                              part + blockIdx.x, part + nbt + blockIdx.x, lsum, yacc_in,
                              yacc_out, last, prod_dyn, lds);
@@ -310,8 +319,9 @@ int launch_spmv_combine(hipStream_t s, long long rows, int np, const double* ypa
 __global__ __launch_bounds__(kBlock) void k_reduce(int nblk, const double* __restrict__ part,
                                                    double* __restrict__ out,
                                                    const int* nval_p, int per, Gate gate) {
-  if (gate.off()) return;
-  if (nval_p && static_cast<int>(blockIdx.x) >= *nval_p * per) return;
+  int nval;
+  if (gated(gate, nval_p, 0, nval)) return;
+  if (nval_p && static_cast<int>(blockIdx.x) >= nval * per) return;
   __shared__ double lds[kBlock / kWave];
   const double v = reduce_partials(part + static_cast<size_t>(blockIdx.x) * nblk, nblk, lds);
   if (threadIdx.x == 0) out[blockIdx.x] = v;
@@ -331,8 +341,8 @@ __global__ __launch_bounds__(kBlock) void k_gemvt(long long L, const T* __restri
                                                   int ncols_v, const int* ncols_p,
                                                   const T* __restrict__ w,
                                                   double* __restrict__ part, Gate gate) {
-  if (gate.off()) return;
-  const int ncols = ncols_p ? *ncols_p : ncols_v;
+  int ncols;
+  if (gated(gate, ncols_p, ncols_v, ncols)) return;
   __shared__ double lds[2][(kBlock / kWave) * kCT];
   gemvt_body<T>(blockIdx.x, L, V, ldv, cols, ncols, w, part, gridDim.x, blockIdx.x, lds);
 }
@@ -356,8 +366,8 @@ __global__ __launch_bounds__(kBlock) void k_gemv_update(long long L, const T* __
                                                         T* __restrict__ w,
                                                         double* __restrict__ part,
                                                         Gate gate) {
-  if (gate.off()) return;
-  const int ncols = ncols_p ? *ncols_p : ncols_v;
+  int ncols;
+  if (gated(gate, ncols_p, ncols_v, ncols)) return;
   __shared__ double lds[kBlock / kWave];
   gemv_update_body<T>(blockIdx.x, L, V, ldv, cols, h, ncols, w, part + blockIdx.x, lds);
 }
@@ -471,7 +481,8 @@ __global__ __launch_bounds__(kBlock) void k_ctl(LbdCtl* __restrict__ gc, char* g
   __shared__ LbdCtlLds c;
   __shared__ LbdCtlRef cg;
   __shared__ double lds[(kBlock / kWave) * 3];
-  if (gc->phase != want_phase || gc->j != want_j) return;
+  const int ph = gc->phase, jj = gc->j;
+  if ((ph != want_phase) | (jj != want_j)) return;
   const bool three = kind >= CTL_ZV_SPMV;
   const bool two = three || (kind != CTL_V_REO && kind != CTL_U_REO);
   ctl_stage_body(gc, garr, cap, want_j, kind, part, nb, two ? part + nb : nullptr, nb, c, cg,

@@ -643,13 +643,25 @@ struct Gate {
   const LbdCtl* c = nullptr;
   int phase = 0, j = 0;
   int flag = 0;  // 0 none, 1 vscale, 2 uscale
+  // One round of loads: tests in turn make each word of the state a memory
+  // round trip of its own at the start of every kernel of a chain.
   __device__ __forceinline__ bool off() const {
     if (!c) return false;
-    if (c->phase != phase || c->j != j) return true;
-    if (flag == 1) return c->vscale == 0;
-    if (flag == 2) return c->uscale == 0;
-    return false;
+    const int ph = c->phase, jj = c->j, vs = c->vscale, us = c->uscale;
+    return (ph != phase) | (jj != j) | ((flag == 1) & (vs == 0)) | ((flag == 2) & (us == 0));
   }
 };
+
+// The gate together with a count that is in device memory (p) or the argument
+// v: both load in one round trip.  True: off.
+__device__ __forceinline__ bool gated(const Gate& gate, const int* p, int v, int& n) {
+  n = v;
+  if (!p) return gate.off();
+  const int m = *p;
+  const bool off = gate.off();
+  ready(m);
+  n = m;
+  return off;
+}
 
 }  // namespace pk

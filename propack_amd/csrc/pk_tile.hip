@@ -76,10 +76,12 @@ __global__ __launch_bounds__(kTB) void k_spmv_tile(
     const unsigned* __restrict__ wd, const VT* __restrict__ va, const T* __restrict__ x,
     T* __restrict__ y, const T* __restrict__ yprev, Scal coef, double* __restrict__ part,
     double* __restrict__ ypart, long long rows, int last, Gate gate) {
-  if (gate.off()) return;
+  const TileDesc t = desc[blockIdx.x];
+  const bool off = gate.off();
+  ready(t.b0);
+  if (off) return;
   extern __shared__ double acc[];
   __shared__ double lds[(kTB / kWave) * 2];
-  const TileDesc t = desc[blockIdx.x];
   const int ng = t.nb / U;  // groups of U batches; at least one
   const unsigned* __restrict__ w0 = wd + static_cast<long long>(t.b0) * kTB + threadIdx.x;
   const VT* __restrict__ v0 = va + static_cast<long long>(t.b0) * kTB + threadIdx.x;
