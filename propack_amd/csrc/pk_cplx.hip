@@ -41,6 +41,7 @@ namespace {
 constexpr int kZRPT = 4;                   // rows per thread of the streaming kernels
 constexpr int kZRows = kBlock * kZRPT;     // rows per workgroup slice
 constexpr int kZCols = 4;                  // basis columns per pass of the Gram-Schmidt kernels
+constexpr int kZProjBlocks = 1024;         // column_groups of the projection (slices of 1024 rows)
 
 template <typename R>
 struct V2T;
@@ -329,6 +330,7 @@ __global__ __launch_bounds__(kBlock) void k_zgemvt(long long L,
   __shared__ double lds[(kBlock / kWave) * 2 * kZCols];
   const size_t nb = gridDim.x;
   if (L <= 0) {  // empty vectors: zero projections, no loads
+    if (blockIdx.y > 0) return;
     for (int j = threadIdx.x; j < 2 * ncols; j += kBlock) part[j * nb + blockIdx.x] = 0.0;
     return;
   }
@@ -343,7 +345,9 @@ __global__ __launch_bounds__(kBlock) void k_zgemvt(long long L,
     wr[r] = row < L ? static_cast<double>(wv.x) : 0.0;
     wi[r] = row < L ? static_cast<double>(wv.y) : 0.0;
   }
-  for (int j0 = 0; j0 < ncols; j0 += kZCols) {
+  int mine;
+  const int first = column_group(ncols, kZCols, blockIdx.y, gridDim.y, mine);
+  for (int j0 = first; j0 < first + mine; j0 += kZCols) {
     C2 a[kZCols][kZRPT];
 #pragma unroll
     for (int q = 0; q < kZCols; ++q) {
@@ -504,8 +508,9 @@ int launch_zgemvt(hipStream_t s, long long L, const void* V, long long ldv, cons
                   int ncols, const int* ncols_p, const void* w, double* part, Gate gate) {
   using C2 = typename V2T<R>::type;
   const int nblk = zstream_blocks(L);
-  hipLaunchKernelGGL(k_zgemvt<R>, dim3(nblk), dim3(kBlock), 0, s, L, static_cast<const C2*>(V),
-                     ldv, cols, ncols, ncols_p, static_cast<const C2*>(w), part, gate);
+  hipLaunchKernelGGL(k_zgemvt<R>, dim3(nblk, column_groups(nblk, ncols, kZCols, kZProjBlocks)),
+                     dim3(kBlock), 0, s, L, static_cast<const C2*>(V), ldv, cols, ncols, ncols_p,
+                     static_cast<const C2*>(w), part, gate);
   return hipGetLastError() == hipSuccess ? nblk : -1;
 }
 

@@ -344,15 +344,17 @@ __global__ __launch_bounds__(kBlock) void k_gemvt(long long L, const T* __restri
   int ncols;
   if (gated(gate, ncols_p, ncols_v, ncols)) return;
   __shared__ double lds[2][(kBlock / kWave) * kCT];
-  gemvt_body<T>(blockIdx.x, L, V, ldv, cols, ncols, w, part, gridDim.x, blockIdx.x, lds);
+  const int c0 = column_group(ncols, kCT, blockIdx.y, gridDim.y, ncols);
+  gemvt_body<T>(blockIdx.x, L, V, ldv, cols + c0, ncols, w,
+                part + static_cast<long long>(c0) * gridDim.x, gridDim.x, blockIdx.x, lds);
 }
 
 template <typename T>
 int launch_gemvt(hipStream_t s, long long L, const T* V, long long ldv, const int* cols,
                  int ncols, const int* ncols_p, const T* w, double* part, Gate gate) {
   const int nblk = cgs_blocks(L);
-  hipLaunchKernelGGL(k_gemvt<T>, dim3(nblk), dim3(kBlock), 0, s, L, V, ldv, cols, ncols,
-                     ncols_p, w, part, gate);
+  hipLaunchKernelGGL(k_gemvt<T>, dim3(nblk, column_groups(nblk, ncols, kCT)), dim3(kBlock), 0, s,
+                     L, V, ldv, cols, ncols, ncols_p, w, part, gate);
   return hipGetLastError() == hipSuccess ? nblk : -1;
 }
 
