@@ -71,11 +71,18 @@ def measured_traffic(kclass, panels, lanes, sort=(0, 0)):
     these shifts the same panels and caps at other shifts answer; None if
     the layout was not measured."""
     want = (*tuple(panels), *tuple(lanes), *tuple(sort))
+    # a negative cap: the tile layout, whatever the panels and the cap
+    tile = sort[0 if kclass == "spmv_n" else 1] <= -1024
     same_bytes = None
     try:
         with open(TRAFFIC_PROFILE) as f:
             for line in f:
                 w = line.split()
+                if tile:
+                    if len(w) == 4 and w[:2] == ["traffic_bytes_per_application", kclass] \
+                            and w[3] == "tile":
+                        return float(w[2])
+                    continue
                 if len(w) not in (7, 9) or w[0] != "traffic_bytes_per_application" \
                         or w[1] != kclass:
                     continue

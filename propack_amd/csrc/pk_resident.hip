@@ -364,7 +364,8 @@ static int resident_grid(const CsrOp* op) {
 
 bool resident_fits(const Engine* e) {
   const CsrOp* op = e->op;
-  // (a host without an operator, and complex bases, run the host executor)
+  // (an engine without an operator runs the host executor, complex bases their
+  // chains)
   if (!op || !e->rbar || (e->prec != PK_F64 && e->prec != PK_F32)) return false;
   for (const CsrOp::Dir* D : {&op->da, &op->dt})
     if (D->sorted || D->tile.nunit > 0 || D->np != 1 || D->pan[0].part.nlong > 0 ||
