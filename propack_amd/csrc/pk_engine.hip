@@ -1106,6 +1106,11 @@ int engine_lanbpro_prepare(Engine* e, int k0, double rnorm) {
 
 int engine_lanbpro_begin(Engine* e, int k0, int k, double* alpha, double* beta, double* rnorm,
                          double* doption, const int* ioption, int* ierr, bool* finished) {
+  // an estimate in flight belongs to this call alone, however it ends
+  struct Taken {
+    Engine* e;
+    ~Taken() { e->u0_started = false; }
+  } taken{e};
   if (k > e->kmax || k0 < 0 || k0 > k) {
     set_error("lanbpro: k=%d k0=%d outside the engine's kmax=%d", k, k0, e->kmax);
     return PK_ERR_ARG;
@@ -1114,13 +1119,11 @@ int engine_lanbpro_begin(Engine* e, int k0, int k, double* alpha, double* beta, 
     set_error("batched steps take real engines only");
     return PK_ERR_NOTSUP;
   }
-  const int rc = e->prec == PK_F64
-                     ? Impl<double>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption,
-                                                     ierr, finished)
-                     : Impl<float>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption,
-                                                    ierr, finished);
-  e->u0_started = false;
-  return rc;
+  if (e->prec == PK_F64)
+    return Impl<double>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption, ierr,
+                                         finished);
+  return Impl<float>(e).lanbpro_begin(k0, k, alpha, beta, rnorm, doption, ioption, ierr,
+                                      finished);
 }
 
 // ||U(:,1)|| of a real engine in two halves: the kernels and the copy
