@@ -81,6 +81,17 @@ __device__ __forceinline__ void spmv_rows_load(RowPre& R, int it0, int r0, int r
   }
 }
 
+// Products of a row that a lane has in flight from LDS (they are added in the
+// same order whatever the depth).  One read and one add after another, a row
+// of 1024 nonzeros on two lanes was 512 LDS round trips, and a launch took as
+// long as its longest row: 20000 x 10000 power law, 98k nonzeros, A x in FP64
+// 22.2 us one at a time, 13.0 four, 10.6 eight; in FP32 26.1, 13.7, 11.3.
+// Eight cost 14 registers: in FP64 they pay on rows of 16 too (200000 x 100000,
+// 3.2M nonzeros: 22.9, 22.9, 22.1), in FP32 four are the faster there (21.3,
+// 21.3, 22.1).
+template <typename T>
+constexpr int kRowDepth = sizeof(T) == 4 ? 4 : 8;
+
 // Row sums of rows [r0, r1) from their products in LDS (prod[q] for the
 // block's q-th nonzero in row-major order): groups of G lanes, lane l of a
 // row adds prod[a + l], prod[a + l + G], ... then a shuffle tree; then the
@@ -111,8 +122,17 @@ __device__ __forceinline__ void spmv_rows(int r0, int r1, int p0, const int* __r
       const int r = r0 + group + (it0 + u) * ngroups;
       const bool valid = r < r1;
       double acc = 0.0;
-      if (valid)
-        for (int q = R.a[u] + lane; q < R.b[u]; q += G) acc += prod[q];
+      if (valid) {
+        int q = R.a[u] + lane;
+        for (; q + (kRowDepth<T> - 1) * G < R.b[u]; q += kRowDepth<T> * G) {
+          double t[kRowDepth<T>];
+#pragma unroll
+          for (int k = 0; k < kRowDepth<T>; ++k) t[k] = prod[q + k * G];
+#pragma unroll
+          for (int k = 0; k < kRowDepth<T>; ++k) acc += t[k];
+        }
+        for (; q < R.b[u]; q += G) acc += prod[q];
+      }
       acc = group_sum<G>(acc);
       if (valid && lane == 0) {
         if (yacc_in) acc = R.yin[u] + acc;

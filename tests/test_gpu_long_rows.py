@@ -48,3 +48,30 @@ def test_long_rows(prec, kw, lengths):
             # both sums in FP64, (count + 2) roundings each, and the store
             bound = 2 * (count + 2) * 2.0 ** -53 * mass + u * (np.abs(want) + mass * 2.0 ** -40)
             assert np.all(np.abs(got.astype(np.float64) - want) <= bound)
+
+
+@pytest.mark.parametrize("prec", [api.PK_F64, api.PK_F32])
+@pytest.mark.parametrize("empty", [1, 60])  # mean rows of about 90 and 3: many lanes a row, few
+@pytest.mark.parametrize("kw", [dict(lanes=(s, s)) for s in range(-2, 3)]
+                         + [dict(sort=(2048, 2048))])
+def test_row_depth(prec, kw, empty):
+    """Rows whose nonzeros per lane lie around the depths that a lane reads
+    at a time (4 and 8), on 2 to 64 lanes a row, beside empty rows: whole
+    numbers small enough that every product and sum is exact."""
+    lengths = sorted({min(max(g * d + e, 0), 1024) for g in (2, 4, 8, 16, 32, 64)
+                      for d in (1, 3, 4, 5, 7, 8, 9, 15, 16, 17) for e in (-1, 0, 1)})
+    g = np.random.default_rng(5)
+    rows = []
+    for length in lengths:
+        rows.append(np.sort(g.choice(4099, length, replace=False)))
+        rows += [np.zeros(0, np.int64)] * empty
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    dt = np.float64 if prec == api.PK_F64 else np.float32
+    A = synth.Csr(len(rows), 4099, rp, np.concatenate(rows).astype(np.int32),
+                  g.integers(-15, 16, int(rp[-1])).astype(dt))
+    for B, trans in ((A, "n"), (A.transpose(), "t")):  # these rows in A, then in A^T
+        op = api.CsrOperator(B, prec, **kw)
+        x = g.integers(-15, 16, A.n).astype(dt)
+        r = np.repeat(np.arange(A.m), np.diff(A.rowptr))
+        want = np.bincount(r, A.val.astype(np.float64) * x.astype(np.float64)[A.col], A.m)
+        assert np.array_equal(op.spmv(x, trans).astype(np.float64), want)
