@@ -7,6 +7,18 @@
 
 namespace pk {
 
+// The gate together with a count that is in device memory (p) or the argument
+// v: both load in one round trip.  True: off.
+__device__ __forceinline__ bool gated(const Gate& gate, const int* p, int v, int& n) {
+  n = v;
+  if (!p) return gate.off();
+  const int m = *p;
+  const bool off = gate.off();
+  ready(m);
+  n = m;
+  return off;
+}
+
 // Partial-sum buffer layout: part[v * nblk + b] for value v of block b.
 // stream_blocks(L) is the fixed grid every streaming kernel over L rows uses;
 // cgs_blocks(L) the grid of the Gram-Schmidt kernels (larger row slices).

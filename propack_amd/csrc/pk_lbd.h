@@ -652,16 +652,4 @@ struct Gate {
   }
 };
 
-// The gate together with a count that is in device memory (p) or the argument
-// v: both load in one round trip.  True: off.
-__device__ __forceinline__ bool gated(const Gate& gate, const int* p, int v, int& n) {
-  n = v;
-  if (!p) return gate.off();
-  const int m = *p;
-  const bool off = gate.off();
-  ready(m);
-  n = m;
-  return off;
-}
-
 }  // namespace pk
