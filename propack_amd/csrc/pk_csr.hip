@@ -105,7 +105,8 @@ int choose_lpr(long long nnz, int rows, int shift = 0) {
 // (1.8M, 70) 29.6 -> 26.6, of another 1M x 500k (4.8M, 342 long rows, half of
 // them under 2048) 106.9 -> 107.1.  Parts of 1024 and more: 33.4, 28.5 and
 // 114.8; of 8192 and more: 38.7, 27.7, 108.8; the chunks ahead of the row
-// blocks: 36.1, 26.7, 108.8.
+// blocks: 36.1, 26.7, 108.8.  These with the row sums one product at a time;
+// with kRowDepth of them in flight the kept cut takes 33.1, 24.2 and 95.2.
 struct Partition {
   std::vector<int4> desc, ldesc;
   int nchunks = 0;
